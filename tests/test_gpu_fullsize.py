@@ -36,10 +36,19 @@ def _rel(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
+def _library_or_skip(name):
+    """a library generated from the reference checkout's model files"""
+    import os
+    from opendihu_amd.build import LIB_DIR
+    if not os.path.exists(os.path.join(LIB_DIR, name)):
+        pytest.skip(f"{name} not built (needs the reference checkout at build time)")
+
+
 @pytest.mark.parametrize("thomas", ["serial", "partitioned"])
 def test_shorten_1024x1481_sampled_fibres(thomas):
     from opendihu_amd.fibers import FiberBatch
     from opendihu_amd.build import SHORTEN_LIBRARY
+    _library_or_skip(SHORTEN_LIBRARY)
     dt, steps = 2.5e-5, 300
     mesh, stim = c2(rate_hz=4000.0)   # the benchmark's batch, motor units firing often
     fibres = [0, 389, 1023]
@@ -123,6 +132,7 @@ def test_hh_4096_uneven_sampled_fibres():
 def test_mixed_16384_sampled_fibres_vs_fp64():
     from opendihu_amd.fibers import FiberBatch
     from opendihu_amd.build import SHORTEN_LIBRARY
+    _library_or_skip(SHORTEN_LIBRARY)
     dt, steps = 2.5e-5, 200
     mesh, stim = c5()
     fibres = [0, 5000, 16383]
@@ -158,6 +168,7 @@ def test_shorten_1024x1481_bench_schedule_1ms():
     fibres against the oracle, Vm within 1e-10 (relative L2) and spike steps equal"""
     from opendihu_amd.fibers import FiberBatch
     from opendihu_amd.build import SHORTEN_LIBRARY
+    _library_or_skip(SHORTEN_LIBRARY)
     import cases
     dt, steps = 2.5e-5, 40000
     mesh, stim = c2(rate_hz=400.0)
