@@ -56,6 +56,8 @@ template <> struct ExpDeriv<ExpLibm> {
     return v;
   }
 };
+template <> struct ExpDeriv<ExpApproxFma> : ExpDeriv<ExpApprox> {};
+template <> struct ExpDeriv<ExpLibmFma> : ExpDeriv<ExpLibm> {};
 
 // u(x) = x / (E(x) - 1) has a removable singularity at x = 0: the HH rates
 // alpha_m = u(-(V+50)/10) and alpha_n = u(-(V+65)/10) / 10. The quotient rule

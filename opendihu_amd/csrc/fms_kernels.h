@@ -25,6 +25,7 @@
 #pragma once
 
 #include "fms_math.h"
+#include "model_hh_fma.h"
 #include <stdint.h>
 
 namespace fms {
@@ -94,6 +95,10 @@ struct DevStim {
 template <class M, class G, class E, bool ALG = false>
 FMS_HD void heun_node(double &V, G *g, const double *p, double t, double dt, bool clamp, double vstim,
                       double *alg_out = nullptr) {
+  if constexpr (std::is_same<M, ModelHH>::value && is_fma<E>::value) {
+    hh_step_fused<G, E, ALG>(V, g, p, dt, clamp, vstim, alg_out);
+    return;
+  }
   // the rates are evaluated in FD (FP64, divisions via div_normal)
   FD y[M::NS], r[M::NS], ys[M::NS], rs[M::NS], a[M::NA], as[M::NA], pp[M::NP > 0 ? M::NP : 1];
 #pragma unroll
@@ -583,15 +588,6 @@ __global__ __launch_bounds__(64) void k_thomas_serial(DevFibers fb, double *vm, 
 // GIVEN_RHS: lv holds the right-hand side itself (adjoint solves) instead of the
 // Vm from which the right-hand side B*Vm is assembled.
 // ----------------------------------------------------------------------------
-// 1/b by the hardware reciprocal and two Newton steps (within about one ulp,
-// not correctly rounded): the partitioned solve is held to a tolerance against
-// the serial recurrence, not to its bits, and multiplies by reciprocals
-__device__ __forceinline__ double recip_nr(double b) {
-  const double r0 = __builtin_amdgcn_rcp(b);
-  const double r1 = __builtin_fma(r0, __builtin_fma(-b, r0, 1.0), r0);
-  return __builtin_fma(r1, __builtin_fma(-b, r1, 1.0), r1);
-}
-
 template <int T, int MMAX, bool GIVEN_RHS = false>
 __device__ __forceinline__ void lds_thomas_part(double *lv, int n, const double *h, double prefactor, double dt,
                                                 bool ie, double *red, int tid) {

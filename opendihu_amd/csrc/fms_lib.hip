@@ -523,7 +523,7 @@ std::vector<unsigned char> graph_signature(const FmsSolver *s, int gsteps, int n
   k.thomas = s->thomas; k.scheme = s->scheme; k.nmax = s->nmax;
   k.pair = s->tune_pair; k.per_fibre = s->tune_reaction_fibre; k.rthreads = s->tune_reaction_threads;
   k.g_is_double = std::is_same<G, double>::value;
-  k.e_is_approx = std::is_same<E, fms::ExpApprox>::value;
+  k.e_is_approx = std::is_base_of<fms::ExpApprox, E>::value;
   std::vector<unsigned char> sig(sizeof(fb) + sizeof(st) + sizeof(k));
   memcpy(sig.data(), &fb, sizeof(fb));
   memcpy(sig.data() + sizeof(fb), &st, sizeof(st));
@@ -700,16 +700,26 @@ int run(FmsSolver *s, const double *h_steps, int K, int n0D, bool fused_only) {
   return 0;
 }
 
+// calls fn with the exponential policy of the solver's runs. Runs with the
+// partitioned solve of a small model are held to a tolerance and take the fused
+// multiply-add forms; the serial solve's runs give the oracle's bits.
+template <class Fn> int with_exp(FmsSolver *s, Fn fn) {
+  const bool approx = s->exp_mode == FMS_EXP_APPROXIMATE;
+  if constexpr (Model::NS <= 8) {
+    if (s->thomas == FMS_THOMAS_PARTITIONED) return approx ? fn(fms::ExpApproxFma{}) : fn(fms::ExpLibmFma{});
+  }
+  return approx ? fn(fms::ExpApprox{}) : fn(fms::ExpLibm{});
+}
+
 int dispatch(FmsSolver *s, const double *h_steps, int K, int n0D) {
   if (K <= 0) return 0;
   if (n0D < 1) return fail(FMS_ERR_ARGUMENT, "n0D must be >= 1");
   if (ensure_flags(s, n0D)) return FMS_ERR_HIP;
-  if (s->precision == FMS_FP64) {
-    if (s->exp_mode == FMS_EXP_APPROXIMATE) return run<double, fms::ExpApprox>(s, h_steps, K, n0D);
-    return run<double, fms::ExpLibm>(s, h_steps, K, n0D);
-  }
-  if (s->exp_mode == FMS_EXP_APPROXIMATE) return run<float, fms::ExpApprox>(s, h_steps, K, n0D);
-  return run<float, fms::ExpLibm>(s, h_steps, K, n0D);
+  return with_exp(s, [&](auto e) {
+    using E = decltype(e);
+    if (s->precision == FMS_FP64) return run<double, E>(s, h_steps, K, n0D);
+    return run<float, E>(s, h_steps, K, n0D);
+  });
 }
 
 size_t gate_bytes(const FmsSolver *s) { return s->precision == FMS_FP64 ? sizeof(double) : sizeof(float); }
@@ -1660,8 +1670,7 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
 }
 
 int adjoint_backward(FmsSolver *s, const double *d_dtraces) {
-  return s->exp_mode == FMS_EXP_APPROXIMATE ? adjoint_backward_core<fms::ExpApprox>(s, d_dtraces)
-                                            : adjoint_backward_core<fms::ExpLibm>(s, d_dtraces);
+  return with_exp(s, [&](auto e) { return adjoint_backward_core<decltype(e)>(s, d_dtraces); });
 }
 
 // forward over all segments, checkpointing; traces go to device memory d_traces
@@ -1718,10 +1727,9 @@ int adjoint_forward(FmsSolver *s, const double *steps, int n_steps, int n0D, int
     tr.sensor_slot = s->d_sensor_slot;
     tr.trace = d_traces + (size_t)k0 * F * S;
     tr.n_sensors = S;
-    if (s->exp_mode == FMS_EXP_APPROXIMATE)
-      rc = launch_fused<double, fms::ExpApprox>(s, s->d_steps + 4 * (size_t)k0, kc, n0D, tr);
-    else
-      rc = launch_fused<double, fms::ExpLibm>(s, s->d_steps + 4 * (size_t)k0, kc, n0D, tr);
+    rc = with_exp(s, [&](auto e) {
+      return launch_fused<double, decltype(e)>(s, s->d_steps + 4 * (size_t)k0, kc, n0D, tr);
+    });
     if (rc) return rc;
   }
   s->adj_whole = whole;

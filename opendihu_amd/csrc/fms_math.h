@@ -12,6 +12,7 @@
 #pragma once
 
 #include <math.h>
+#include <type_traits>
 
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
@@ -112,6 +113,28 @@ struct ExpLibm {
   static FMS_HD FD exp(FD x) { return FD(::exp(x.v)); }
   static FMS_HD FD log(FD x) { return FD(::log(x.v)); }
 };
+
+// The same two exponentials in the runs held to a tolerance instead of to the
+// oracle's bits (partitioned solve): a model that has a fused form of its
+// reaction (hh_step_fused in model_hh_fma.h) takes it under these policies, every
+// other model computes as under their bases.
+struct ExpApproxFma : ExpApprox {};
+struct ExpLibmFma : ExpLibm {};
+template <class E> struct is_fma : std::false_type {};
+template <> struct is_fma<ExpApproxFma> : std::true_type {};
+template <> struct is_fma<ExpLibmFma> : std::true_type {};
+
+// 1/b by the hardware reciprocal and two Newton steps (within about one ulp,
+// not correctly rounded), for results held to a tolerance
+FMS_HD double recip_nr(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double r0 = __builtin_amdgcn_rcp(b);
+  const double r1 = __builtin_fma(r0, __builtin_fma(-b, r0, 1.0), r0);
+  return __builtin_fma(r1, __builtin_fma(-b, r1, 1.0), r1);
+#else
+  return 1.0 / b;
+#endif
+}
 
 // Natural logarithm from IEEE double operations only (no library call beyond
 // the exact frexp), so that a C build with the same operations returns the
