@@ -14,6 +14,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_DIR = os.path.dirname(PKG_DIR)
@@ -29,7 +31,7 @@ ARCH = os.environ.get("FMS_OFFLOAD_ARCH", "gfx950")
 # g++ -std=c++17 build of its generated code (bit-exact parity).
 # -packed-fp32-ops: no packed FP32 instructions are generated.
 HIP_FLAGS = [
-    f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
+    f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
@@ -43,6 +45,7 @@ HIP_FLAGS = [
 # scheduler, which is faster for them (occupancy matters there).
 LARGE_MODEL_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 LARGE_MODEL_STATES = 8
+SMALL_MODEL_PARTS = 6   # FMS_PART values of fms_parts.hip
 
 HH_LIBRARY = "libfms_hodgkin_huxley_1952.so"
 
@@ -72,10 +75,18 @@ def compile_library(out_name: str, model_header: str | None = None, model_type: 
         cmd.append(f"-I{extra_include}")
     if model_header:
         cmd += [f'-DFMS_MODEL_HEADER="{model_header}"', f"-DFMS_MODEL_TYPE={model_type}"]
-    tmp = out + ".tmp"
-    cmd += ["-o", tmp, os.path.join(CSRC, "fms_lib.hip")]
-    _run(cmd)
-    os.replace(tmp, out)
+    # the host runtime, and the small models' large kernels in objects of their own
+    # (fms_parts.h), one compiler process each
+    parts = SMALL_MODEL_PARTS if n_states <= LARGE_MODEL_STATES else 0
+    with tempfile.TemporaryDirectory(dir=LIB_DIR) as tmp:
+        jobs = [[os.path.join(CSRC, "fms_lib.hip"), "-o", os.path.join(tmp, "lib.o")]]
+        jobs += [[f"-DFMS_PART={k}", os.path.join(CSRC, "fms_parts.hip"), "-o", os.path.join(tmp, f"part{k}.o")]
+                 for k in range(parts)]
+        with ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
+            list(ex.map(lambda j: _run([*cmd, "-c", *j]), jobs))
+        built = os.path.join(tmp, out_name)
+        _run([HIPCC, f"--offload-arch={ARCH}", "-fPIC", "-shared", "-o", built, *[j[-1] for j in jobs]])
+        os.replace(built, out)
     return out
 
 
@@ -152,7 +163,6 @@ def build_vc_kernel_library(kernel_file: str, name: str, lib_name: str, ilp_sche
 def build_reference_models(reference_root: str) -> list[str]:
     """Libraries for the CellML models shipped in the reference's test inputs
     (compiled concurrently, one hipcc process per model)."""
-    from concurrent.futures import ThreadPoolExecutor
     jobs = [(os.path.join(reference_root, rel), pa, pc, name, lib)
             for rel, name, pa, pc, lib in REFERENCE_MODELS if os.path.exists(os.path.join(reference_root, rel))]
     vc_jobs = [(os.path.join(reference_root, rel), name, lib, ilp)

@@ -396,7 +396,7 @@ __global__ __launch_bounds__(T) void k_adj_fused(DevFibers fb, DevStim st, const
 }
 
 // per-fibre sums of the per-node parameter-gradient accumulators
-__global__ void k_adj_reduce(DevFibers fb, const double *gacc, double *grad) {
+static __global__ void k_adj_reduce(DevFibers fb, const double *gacc, double *grad) {
   const int f = blockIdx.x;
   const int off = fb.fiber_off[f], n = fb.fiber_off[f + 1] - off;
   __shared__ double part[3][256];

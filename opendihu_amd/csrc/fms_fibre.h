@@ -1,0 +1,336 @@
+// Resident fused kernel of the small models (at most 8 states, partitioned
+// solve): one workgroup per fibre runs many split steps with the whole state of
+// the fibre in registers.
+//
+//  * Thread t owns the c = ceil(n / T) consecutive nodes from t*c on, for the
+//    reaction and for the diffusion (fms_chunk.h) alike: Vm and gates never leave
+//    its registers between two launches, and the diffusion's coefficients stay
+//    beside them as long as dt does not change. One barrier per split step.
+//  * Waves past the fibre's end skip the reaction; threads past it shadow its
+//    last node and store nothing.
+//  * Nodes are advanced two at a time (two independent chains per instruction
+//    stream); the Heun step with a stimulus is a second copy of that code, taken
+//    by the waves that hold stimulated nodes while the stimulus is on.
+//  * The stimulation state machine does not depend on the states: k_fibre_flags
+//    evaluates it for the whole launch beforehand, one wave per fibre, 64 Heun
+//    steps at a time.
+//
+// Bound by FP64 instruction issue: the two reaction halves are about 450
+// instructions per node and step, the solve about 15.
+#pragma once
+
+#include "fms_chunk.h"
+#include "fms_fused.h"
+
+namespace fms {
+
+// flags of 64 consecutive Heun steps of one fibre (per split step the n0D of the
+// first half, then the n0D of the second): bit i of `stim` says whether the
+// stimulus is on, of `compute` whether the reaction runs
+struct FlagGroup {
+  unsigned long long stim, compute;
+};
+
+__host__ __device__ constexpr long long flag_groups(long long steps, int n0D) { return (steps * 2 * n0D + 63) / 64; }
+
+// The state machine of stim_flag for the K split steps from `steps` on, one wave
+// per fibre. Lane i evaluates Heun step i of each group of 64 against the state
+// machine's current state; at the first lane whose check changes that state
+// (repeat time over: next period, next jitter value) the lanes before it are
+// final, the state advances and the lanes after it are evaluated again: the same
+// checks on the same values as one thread going through the steps in time order,
+// whose chain of global loads per step the fused kernel had waited for.
+static __global__ __launch_bounds__(64) void k_fibre_flags(DevStim st, const double *__restrict__ steps, int K, int n0D,
+                                                    FlagGroup *__restrict__ flags) {
+  const int f = blockIdx.x, lane = threadIdx.x;
+  const long long count = (long long)K * 2 * n0D, groups = flag_groups(K, n0D);
+  FlagGroup *out = flags + f * groups;
+  const bool only = st.only_if_stimulated != 0;
+  bool hb = st.has_been[f] != 0;
+  const bool hb_start = hb;
+  const bool table = st.mode == 1;
+  double freq = 0, repeat = 0, begin = 0, last = 0, jit = 0, onset = 0, duration = 0;
+  int col = 0, jidx = 0, currently = 0;
+  if (table) {
+    freq = st.freq[f];
+    repeat = st.repeat[f];
+    begin = st.enable_begin[f];
+    col = st.motor_unit[f] % st.fe_cols;
+    last = st.last_check[f];
+    jit = st.cur_jitter[f];
+    jidx = st.jitter_idx[f];
+    currently = st.currently[f];
+  }
+  for (long long gi = 0; gi < groups; gi++) {
+    const long long i = gi * 64 + lane;
+    const bool active = i < count;
+    double t = 0.0;
+    if (active) {
+      const long long s = i / (2 * n0D);
+      const int r = (int)(i - s * 2 * n0D);
+      const double *row = steps + 4 * s;
+      t = half_start(row, r / n0D) + (r % n0D) * row[2];
+    }
+    int stim = 0;
+    if (table) {
+      int fires = 0;
+      if (active) {
+        const int idx = (int)round(t * freq);
+        const unsigned long fr = (unsigned long)(long)idx % (unsigned long)st.fe_rows;
+        fires = st.firing_events[fr * st.fe_cols + col];
+      }
+      int done = 0;   // lanes before it are final
+      while (done < 64) {
+        const double next = last + 1. / (freq + jit);
+        const bool due = active && lane >= done && t >= next && t >= begin - 1e-13;
+        const bool change = due && repeat != 0 && t - next > repeat;
+        const unsigned long long mc = __builtin_amdgcn_ballot_w64(change);
+        const int first = mc ? __builtin_ctzll(mc) : 64;
+        if (lane >= done && lane < first) stim = due && fires;
+        if (first < 64) {
+          last += 1. / (freq + jit);
+          double jf = 0.0;
+          if (st.jitter_cnt[f] > 0) jf = st.jitter[st.jitter_off[f] + jidx % st.jitter_cnt[f]];
+          jit = jf * freq;
+          jidx++;
+        }
+        done = first + 1;
+      }
+    } else if (st.mode == 2) {
+      stim = active && current_on(st, f, t);
+    }
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(stim != 0);
+    if (table) {
+      // rising edges: stimulated now and not at the step before
+      const unsigned long long rise = m & ~((m << 1) | (currently ? 1ULL : 0ULL));
+      if (rise && st.log_count) {
+        int k0 = 0;
+        if (lane == 0) k0 = atomicAdd(st.log_count, __builtin_popcountll(rise));
+        k0 = __shfl(k0, 0);
+        const int k = k0 + __builtin_popcountll(rise & ((1ULL << lane) - 1));
+        if (((rise >> lane) & 1) && k < st.log_cap) {
+          st.log_time[k] = t;
+          st.log_fiber[k] = f;
+        }
+      }
+      const int last_lane = count - gi * 64 < 64 ? (int)(count - gi * 64) - 1 : 63;
+      currently = (int)((m >> last_lane) & 1);
+    }
+    // the fibre computes from the Heun step of its first stimulation on
+    const unsigned long long since = m ? ~0ULL << __builtin_ctzll(m) : 0ULL;
+    if (lane == 0) out[gi] = FlagGroup{m, !only || hb ? ~0ULL : since};
+    hb = hb || m != 0;
+  }
+  if (lane == 0) {
+    if (table) {
+      st.last_check[f] = last;
+      st.cur_jitter[f] = jit;
+      st.jitter_idx[f] = jidx;
+      st.currently[f] = (unsigned char)currently;
+    }
+    if (hb && !hb_start) st.has_been[f] = 1;
+  }
+}
+
+// nodes whose Heun steps share a basic block
+#ifndef FIBRE_GROUP
+#define FIBRE_GROUP 1
+#endif
+
+// what the fused kernel needs of the stimulation
+struct FibreStim {
+  int clamp;        // the stimulus sets Vm to vstim (firing table), else parameter `param` to the amplitude
+  int param;
+  double vstim;
+  const double *amplitude;   // [F], current pulses
+  const FlagGroup *flags;    // [F][flag_groups(K, n0D)]
+};
+
+// One Heun step of the thread's nodes. `on`: the stimulus is on and the wave holds
+// stimulated nodes (bits of `inset`); it is uniform over the wave, so the selects it
+// needs cost the other steps a branch.
+template <class M, class G, class E, int C>
+__device__ __forceinline__ void fibre_heun(double *V, G (*g)[M::NS - 1], const double *p, double t, double dt, bool on,
+                                           unsigned inset, const FibreStim &st, double amplitude) {
+  if constexpr (std::is_same<M, ModelHH>::value) {
+    if (!on || st.clamp || st.param == 0) {
+      constexpr_for<0, C, FIBRE_GROUP>([&](auto k_) {
+        constexpr int k = decltype(k_)::value, Q = k + FIBRE_GROUP <= C ? FIBRE_GROUP : C - k;
+        double p0[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++) p0[q] = p[0];
+        if (on && !st.clamp) {
+#pragma unroll
+          for (int q = 0; q < Q; q++) p0[q] = (inset >> (k + q)) & 1 ? amplitude : p[0];
+        }
+        hh_step_nodes<G, E, false, Q>(V + k, g + k, p, p0, dt,
+                                      [&](double(*ys)[4]) {
+                                        if (on && st.clamp) {
+#pragma unroll
+                                          for (int q = 0; q < Q; q++)
+                                            ys[q][0] = (inset >> (k + q)) & 1 ? st.vstim : ys[q][0];
+                                        }
+                                      },
+                                      nullptr);
+        if (on && st.clamp) {
+#pragma unroll
+          for (int q = 0; q < Q; q++) V[k + q] = (inset >> (k + q)) & 1 ? st.vstim : V[k + q];
+        }
+      });
+      return;
+    }
+  }
+  // other models, and a stimulus on another parameter
+  constexpr_for<0, C, 1>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    const bool in = on && ((inset >> k) & 1);
+    double pk[M::NP > 0 ? M::NP : 1];
+#pragma unroll
+    for (int q = 0; q < M::NP; q++) pk[q] = in && !st.clamp && q == st.param ? amplitude : p[q];
+    heun_node<M, G, E, false>(V[k], g[k], pk, t, dt, in && st.clamp, st.vstim);
+  });
+}
+
+// the fibre's steps with C nodes per thread; TAPE: sensor traces and the adjoint's
+// tape are recorded (either may be absent)
+template <class M, class G, class E, int T, int C, bool TAPE>
+__device__ __forceinline__ void fibre_steps(const DevFibers &fb, const FibreStim &st, double *__restrict__ vm,
+                                            G *__restrict__ gates, const double *__restrict__ steps, int K, int n0D,
+                                            int ie, const DevSpikes &spk, const DevTrace &tr, int f, int off, int n,
+                                            double *sh) {
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const double pf = fb.prefactor[f];
+  const ChunkLds<T, C> lds{sh, tid};
+  const int lo = tid * C;
+  const bool busy = wave * 64 * C < n;   // the wave holds nodes of the fibre
+  const FlagGroup *flags = st.flags + f * flag_groups(K, n0D);
+
+  double p[M::NP > 0 ? M::NP : 1];
+#pragma unroll
+  for (int k = 0; k < M::NP; k++) p[k] = fb.params[(long long)f * M::NP + k];
+  double V[C];
+  G g[C][M::NS - 1];
+  unsigned inset = 0, below = 0, sensor = 0;
+  {
+    const int sb = fb.stim_begin[f], se = fb.stim_end[f];
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+      const int i = off + (lo + k < n ? lo + k : n - 1);
+      V[k] = vm[i];
+#pragma unroll
+      for (int q = 0; q < M::NS - 1; q++) g[k][q] = gates[(long long)q * fb.gate_stride + i];
+      if (lo + k < n) {
+        inset |= (lo + k >= sb && lo + k < se ? 1u : 0u) << k;
+        // bit k of `below`: node k was below the threshold at the last check
+        if (spk.enabled) below |= (spk.vm_prev[i] < spk.threshold ? 1u : 0u) << k;
+        if (TAPE && tr.sensor_slot) sensor |= (tr.sensor_slot[i] >= 0 ? 1u : 0u) << k;
+      }
+    }
+  }
+  const bool wave_inset = __builtin_amdgcn_ballot_w64(inset != 0) != 0;
+
+  // half step hs: the first reaction half of step hs / 2, or (odd) its diffusion
+  // and second reaction half. The outer loop runs once per change of dt.
+  int hs = 0;
+  FlagGroup fl{0, 0};
+  while (hs < 2 * K) {
+    const double dt1 = steps[4 * (long long)(hs >> 1) + 3];
+    ChunkFactor<C> fac;
+    chunk_refactor<T, C>(fac, n, fb.elem_len + (off - f), pf, dt1, ie != 0, lds);
+#pragma unroll 1
+    do {
+      const int s = hs >> 1;
+      const bool half = hs & 1;
+      const double *row = steps + 4 * (long long)s;
+      if (half) chunk_diffuse<T, C>(fac, V, s & 1, lds);
+      if (TAPE && tr.tape) {
+        // half 0: the state before it; half 1: Vm after the diffusion
+#pragma unroll
+        for (int k = 0; k < C; k++)
+          if (lo + k < n) {
+            if (half)
+              tape_store<M::NS>(tr, fb.n_total, s, 2 * M::NS, off + lo + k, V[k], g[k], 1);
+            else
+              tape_store<M::NS>(tr, fb.n_total, s, 0, off + lo + k, V[k], g[k], M::NS);
+          }
+      }
+      if (busy) {
+        const double t0 = half_start(row, half), dt = row[2];
+#pragma unroll 1
+        for (int j = 0; j < n0D; j++) {
+          const int q = hs * n0D + j;
+          if ((q & 63) == 0) fl = flags[q >> 6];
+          if (!((fl.compute >> (q & 63)) & 1)) continue;
+          const bool on = wave_inset && ((fl.stim >> (q & 63)) & 1);
+          fibre_heun<M, G, E, C>(V, g, p, t0 + j * dt, dt, on, inset, st, on && !st.clamp ? st.amplitude[f] : 0.0);
+        }
+      }
+      if (TAPE && tr.tape && !half) {
+#pragma unroll
+        for (int k = 0; k < C; k++)
+          if (lo + k < n) tape_store<M::NS>(tr, fb.n_total, s, M::NS, off + lo + k, V[k], g[k], M::NS);
+      }
+      if (half && TAPE && sensor) {
+#pragma unroll
+        for (int k = 0; k < C; k++)
+          if ((sensor >> k) & 1)
+            tr.trace[((long long)s * fb.n_fibers + f) * tr.n_sensors + tr.sensor_slot[off + lo + k]] = V[k];
+      }
+      if (half && spk.enabled && busy) {
+        unsigned now = 0;
+#pragma unroll
+        for (int k = 0; k < C; k++) now |= (V[k] < spk.threshold ? 1u : 0u) << k;
+        // nodes that were below the threshold and are not (a NaN is no crossing)
+        const unsigned cross = below & ~now;
+        below = now;
+        if (cross) {
+#pragma unroll
+          for (int k = 0; k < C; k++)
+            if (((cross >> k) & 1) && lo + k < n && V[k] >= spk.threshold) {
+              const int i = off + lo + k;
+              spk.count[i]++;
+              if (spk.first_step[i] < 0) spk.first_step[i] = spk.step0 + s + 1;
+            }
+        }
+      }
+      hs++;
+    } while (hs < 2 * K && (!(hs & 1) || steps[4 * (long long)(hs >> 1) + 3] == dt1));
+  }
+
+#pragma unroll
+  for (int k = 0; k < C; k++)
+    if (lo + k < n) {
+      const int i = off + lo + k;
+      vm[i] = V[k];
+#pragma unroll
+      for (int q = 0; q < M::NS - 1; q++) gates[(long long)q * fb.gate_stride + i] = g[k][q];
+      // the last check's Vm is the launch's final Vm
+      if (spk.enabled) spk.vm_prev[i] = V[k];
+    }
+}
+
+// waves per SIMD the kernel is compiled for
+template <int T, int CMAX> constexpr int fibre_occupancy() {
+#ifdef FIBRE_OCC
+  return FIBRE_OCC;
+#endif
+  return T >= 512 && CMAX <= 4 ? 4 : 2;
+}
+
+// one workgroup per fibre; its threads take as many nodes each as the fibre needs
+template <class M, class G, class E, int T, int CMAX, bool TAPE>
+__global__ __launch_bounds__(T, (fibre_occupancy<T, CMAX>())) void k_fibre(
+    DevFibers fb, FibreStim st, double *__restrict__ vm, G *__restrict__ gates, const double *__restrict__ steps, int K,
+    int n0D, int ie, const int *__restrict__ order, DevSpikes spk, DevTrace tr) {
+  extern __shared__ double sh[];
+  if (TAPE && tr.raise_priority) __builtin_amdgcn_s_setprio(2);
+  const int f = __builtin_amdgcn_readfirstlane(order[blockIdx.x]);
+  const int off = fb.fiber_off[f];
+  const int n = fb.fiber_off[f + 1] - off;
+  with_chunk_rows<CMAX>((n + T - 1) / T, [&](auto c_) {
+    fibre_steps<M, G, E, T, decltype(c_)::value, TAPE>(fb, st, vm, gates, steps, K, n0D, ie, spk, tr, f, off, n, sh);
+  });
+}
+
+}  // namespace fms

@@ -258,10 +258,10 @@ __global__ __launch_bounds__(T) void k_fused(DevFibers fb, DevStim st, double *_
     const bool more = s + 1 < K;
 
     // diffusion (one solve per split step, as the reference)
-    if (serial) {
+    if (M::NS <= 8 || serial) {   // small models: k_fibre takes the partitioned runs
       if (tid == 0) thomas_serial_fiber(lv, n, h, pf, dt1, ie != 0, red, red + n);
       __syncthreads();
-    } else {
+    } else if constexpr (M::NS > 8) {
       lds_thomas_part<T, MMAX>(lv, n, h, pf, dt1, ie != 0, red, tid);
     }
 

@@ -231,7 +231,7 @@ __device__ __forceinline__ double half_start(const double *row, int half) {
   return half ? row[0] + 0.5 * row[1] : row[0];
 }
 
-__global__ void k_cursor_set(long long *cursor, long long row, long long step_counter, const double *table) {
+static __global__ void k_cursor_set(long long *cursor, long long row, long long step_counter, const double *table) {
   if (threadIdx.x == 0) {
     cursor[0] = row;
     cursor[1] = step_counter;
@@ -239,12 +239,12 @@ __global__ void k_cursor_set(long long *cursor, long long row, long long step_co
   }
 }
 
-__global__ void k_cursor_advance(long long *cursor, int g) {
+static __global__ void k_cursor_advance(long long *cursor, int g) {
   if (threadIdx.x == 0) cursor[0] += g;
 }
 
 // one thread per fibre: flags[f*n0D + j] for the n0D Heun steps of a half step
-__global__ void k_stim_flags(DevStim st, int n_fibers, unsigned char *flags, StepRef sr, int half, int n0D) {
+static __global__ void k_stim_flags(DevStim st, int n_fibers, unsigned char *flags, StepRef sr, int half, int n0D) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= n_fibers) return;
   const double *row = sr.row();
@@ -256,7 +256,7 @@ __global__ void k_stim_flags(DevStim st, int n_fibers, unsigned char *flags, Ste
 // flags of two consecutive reaction halves, the second half of step q and the
 // first half of step q+1, in the state machine's time order: flags[f*n0D + j]
 // and flags[(n_fibers + f)*n0D + j]
-__global__ void k_stim_flags_pair(DevStim st, int n_fibers, unsigned char *flags, StepRef sr, int n0D) {
+static __global__ void k_stim_flags_pair(DevStim st, int n_fibers, unsigned char *flags, StepRef sr, int n0D) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= n_fibers) return;
   const double *row = sr.row();
@@ -551,7 +551,7 @@ FMS_HD void thomas_serial_fiber(double *u, int n, const double *h, double prefac
 }
 
 // one lane per fibre: bit-exact reference recurrence
-__global__ __launch_bounds__(64) void k_thomas_serial(DevFibers fb, double *vm, double *cA, double *dA, StepRef sr,
+static __global__ __launch_bounds__(64) void k_thomas_serial(DevFibers fb, double *vm, double *cA, double *dA, StepRef sr,
                                                       int ie) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= fb.n_fibers) return;
@@ -796,7 +796,7 @@ __global__ __launch_bounds__(256) void k_eval_heun(double *__restrict__ ys, cons
 }
 
 // spike detector: upward crossings of the threshold after each split step
-__global__ void k_spikes(long long N, const double *vm, double *vm_prev, int *first_step, int *count, double th,
+static __global__ void k_spikes(long long N, const double *vm, double *vm_prev, int *first_step, int *count, double th,
                          StepRef sr) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;

@@ -22,14 +22,8 @@
 #include "fms_adjoint.h"
 #include "fms_fused.h"
 #include "fms_kernels.h"
+#include "fms_parts.h"
 
-#ifndef FMS_MODEL_HEADER
-#define FMS_MODEL_HEADER "model_hh.h"
-#define FMS_MODEL_TYPE fms::ModelHH
-#endif
-#include FMS_MODEL_HEADER
-
-using Model = FMS_MODEL_TYPE;
 
 namespace {
 
@@ -119,7 +113,8 @@ struct FmsSolver {
   void *d_gates = nullptr;    // double or float [(NS-1)*GS]
   double *d_cA = nullptr, *d_dA = nullptr;  // serial Thomas scratch (split kernels)
   unsigned char *d_flags = nullptr;
-  int flags_cap = 0;
+  bool noalloc = false;   // the running call may not allocate (fms_advance_schedule_noalloc)
+  size_t flags_cap = 0;   // bytes
   double *d_steps = nullptr;
   int steps_cap = 0;
 
@@ -297,16 +292,19 @@ fms::DevSpikes dev_spikes(const FmsSolver *s) {
   return spk;
 }
 
-// the flags of one reaction half, or of a pair of halves (second buffer half)
-int ensure_flags(FmsSolver *s, int n0D) {
-  if (s->flags_cap < 2 * s->F * n0D) {
+int ensure_flag_bytes(FmsSolver *s, size_t bytes) {
+  if (s->flags_cap < bytes) {
     if (s->d_flags) HIP_TRY(hipFree(s->d_flags));
     s->d_flags = nullptr;
-    s->flags_cap = 2 * s->F * n0D;
-    if (dalloc(&s->d_flags, (size_t)s->flags_cap)) return FMS_ERR_HIP;
+    s->flags_cap = 0;
+    if (dalloc(&s->d_flags, bytes)) return FMS_ERR_HIP;
+    s->flags_cap = bytes;
   }
   return 0;
 }
+
+// the flags of one reaction half, or of a pair of halves (second buffer half)
+int ensure_flags(FmsSolver *s, int n0D) { return ensure_flag_bytes(s, (size_t)2 * s->F * n0D); }
 
 // adds the durations of the recorded launches to their classes
 void prof_drain(FmsSolver *s) {
@@ -356,8 +354,8 @@ struct KernelTimer {
 
 // device step table: the K records of this call plus a copy of the last one
 // (the fused kernel reads one record ahead); the cursor starts at row 0 with
-// the current spike-step counter
-int upload_steps(FmsSolver *s, const double *steps, int K) {
+// the current spike-step counter (the split kernels read it; the others do not)
+int upload_steps(FmsSolver *s, const double *steps, int K, bool cursor = true) {
   if (s->steps_cap < 4 * (K + 1)) {
     if (s->d_steps) HIP_TRY(hipFree(s->d_steps));
     s->d_steps = nullptr;
@@ -367,6 +365,7 @@ int upload_steps(FmsSolver *s, const double *steps, int K) {
   HIP_TRY(hipMemcpyAsync(s->d_steps, steps, 4 * (size_t)K * sizeof(double), hipMemcpyHostToDevice, s->stream));
   HIP_TRY(hipMemcpyAsync(s->d_steps + 4 * (size_t)K, steps + 4 * (size_t)(K - 1), 4 * sizeof(double),
                          hipMemcpyHostToDevice, s->stream));
+  if (!cursor) return 0;
   hipLaunchKernelGGL(fms::k_cursor_set, dim3(1), dim3(64), 0, s->stream, s->d_cursor, 0LL, s->step_counter,
                      (const double *)s->d_steps);
   HIP_TRY(hipGetLastError());
@@ -445,9 +444,39 @@ int launch_flags_pair(FmsSolver *s, int q, int n0D) {
   return 0;
 }
 
+// Threads per fibre of the chunked kernels. Every kernel of the solver takes the
+// same, so that its schedules agree in every bit. A thread owns ceil(n / T) <= 8
+// nodes; 512 only for the fibres that need them: with 256, two fibres share a CU and
+// one's solve hides behind the other's reaction (4096 fibres of 400-2000 nodes: 80
+// against 109 us per step), and with one fibre per CU they differ by a few per cent
+// in either direction (256 x 1000 nodes: both 6.1 us; 16 x 600: 4.6 against 5.3).
+int chunk_threads(const FmsSolver *s) {
+  if (s->tune_threads == 128 && s->nmax <= 1024) return 128;
+  return s->nmax > 2048 ? 512 : 256;
+}
+
+// the models whose partitioned solve is the chunked one
+constexpr bool chunked_model() { return Model::NS <= 8; }
+
+template <int T> void launch_diffuse_chunk(FmsSolver *s, int q, int ie) {
+  const size_t lds = (size_t)(20 * (T / 64) + s->nmax) * sizeof(double);
+  FMS_LAUNCH(s, (fms::k_diffuse_chunk<T, 8>), dim3(s->F), dim3(T), lds, s->fibers(), s->d_vm, step_ref(s, q), ie);
+}
+
 int launch_thomas(FmsSolver *s, int q) {
   KernelTimer timer(s, FMS_KERNEL_DIFFUSION);
   const int ie = s->scheme == FMS_IMPLICIT_EULER;
+  if constexpr (chunked_model()) {
+    if (s->thomas == FMS_THOMAS_PARTITIONED) {
+      const int T = chunk_threads(s);
+      if (T == 128) launch_diffuse_chunk<128>(s, q, ie);
+      else if (T == 512) launch_diffuse_chunk<512>(s, q, ie);
+      else launch_diffuse_chunk<256>(s, q, ie);
+      HIP_TRY(hipGetLastError());
+      s->n_launch_thomas++;
+      return 0;
+    }
+  }
   if (s->thomas == FMS_THOMAS_SERIAL) {
     const int threads = 64;
     FMS_LAUNCH(s, fms::k_thomas_serial, dim3((s->F + threads - 1) / threads), dim3(threads), 0,
@@ -633,20 +662,68 @@ int launch_fused_npt(FmsSolver *s, const double *d_steps, int K, int n0D, const 
   return 0;
 }
 
+// bytes of the flags that one launch of K steps reads
+size_t fibre_flag_bytes(const FmsSolver *s, int K, int n0D) {
+  return (size_t)s->F * fms::flag_groups(K, n0D) * sizeof(fms::FlagGroup);
+}
+
+// the flags of K steps, then the steps
+template <class G, class E, bool TAPE>
+int launch_fibre(FmsSolver *s, const double *d_steps, int K, int n0D, const fms::DevTrace &tr) {
+  {
+    KernelTimer timer(s, FMS_KERNEL_OTHER);
+    FMS_LAUNCH(s, fms::k_fibre_flags, dim3(s->F), dim3(64), 0, s->stim(), d_steps, K, n0D,
+               reinterpret_cast<fms::FlagGroup *>(s->d_flags));
+    HIP_TRY(hipGetLastError());
+  }
+  KernelTimer timer(s, FMS_KERNEL_FUSED);
+  fms::FibreLaunch l{};
+  l.fb = s->fibers();
+  l.st = fms::FibreStim{s->stim_mode == FMS_STIM_FIRING_TABLE, s->stim_param, s->vstim, s->d_amp,
+                        reinterpret_cast<const fms::FlagGroup *>(s->d_flags)};
+  l.vm = s->d_vm;
+  l.gates = s->d_gates;
+  l.steps = d_steps;
+  l.nmax = s->nmax;
+  l.K = K;
+  l.n0D = n0D;
+  l.ie = s->scheme == FMS_IMPLICIT_EULER ? 1 : 0;
+  l.order = s->d_order;
+  l.spk = dev_spikes(s);
+  l.tr = tr;
+  l.stream = s->stream;
+  if (s->prof_slot >= 0) {
+    l.start = s->prof_ev[2 * s->prof_slot];
+    l.stop = s->prof_ev[2 * s->prof_slot + 1];
+    s->prof_launched = 1;
+  }
+  fms::fibre_launch<G, E, TAPE>(chunk_threads(s), l);
+  HIP_TRY(hipGetLastError());
+  s->step_counter += K;
+  s->n_launch_fused++;
+  return 0;
+}
+
 // Fused schedules: one workgroup of T threads per fibre; gates resident in
 // registers (NPT nodes per thread, small models) or streamed from HBM. The
 // partitioned solve needs ceil(n / T) <= MMAX rows per thread, the serial
 // solve 2n <= 16 T doubles of LDS scratch (fms_set_tuning checks both).
 template <class G, class E>
 int launch_fused(FmsSolver *s, const double *d_steps, int K, int n0D, const fms::DevTrace &tr = fms::DevTrace{}) {
+  if constexpr (chunked_model() && fms::is_fma<E>::value) {
+    // sensors and the tape are the adjoint's, which runs in FP64
+    if constexpr (std::is_same<G, double>::value)
+      if (tr.sensor_slot || tr.tape) return launch_fibre<G, E, true>(s, d_steps, K, n0D, tr);
+    return launch_fibre<G, E, false>(s, d_steps, K, n0D, tr);
+  } else {
   const bool resident = s->tune_resident != 0;
   if constexpr (Model::NS <= 8) {
     if (s->tune_threads == 128) {
       // resident gates for at most 8 nodes per thread: 16 per thread spill to
       // scratch, and that build of the fused kernel computed wrong states
       const int npt = (s->nmax + 127) / 128;
-      if (resident && npt <= 8) return launch_fused_npt<G, E, 128, 8, 16>(s, d_steps, K, n0D, tr);
-      return launch_fused_npt<G, E, 128, 0, 16>(s, d_steps, K, n0D, tr);
+      if (resident && npt <= 8) return launch_fused_npt<G, E, 128, 8, 8>(s, d_steps, K, n0D, tr);
+      return launch_fused_npt<G, E, 128, 0, 8>(s, d_steps, K, n0D, tr);
     }
   }
   constexpr int T = FUSED_T;
@@ -657,6 +734,7 @@ int launch_fused(FmsSolver *s, const double *d_steps, int K, int n0D, const fms:
   }
   if (npt <= 8) return launch_fused_npt<G, E, T, 0, 8>(s, d_steps, K, n0D, tr);
   return launch_fused_npt<G, E, T, 0, 16>(s, d_steps, K, n0D, tr);
+  }
 }
 
 template <class G, class E>
@@ -664,8 +742,11 @@ int run(FmsSolver *s, const double *h_steps, int K, int n0D, bool fused_only);
 
 template <class G, class E>
 int run(FmsSolver *s, const double *h_steps, int K, int n0D) {
-  // the point-buffer order decides per node: the per-node split kernels
-  if (s->kernels == FMS_KERNELS_SPLIT || s->vc_width) {
+  // the point-buffer order decides per node: the per-node split kernels. They
+  // also take a call without allocation whose flags of one fused step do not fit.
+  const bool fibre = chunked_model() && fms::is_fma<E>::value;
+  const bool flags_fit = !fibre || !s->noalloc || fibre_flag_bytes(s, 1, n0D) <= s->flags_cap;
+  if (s->kernels == FMS_KERNELS_SPLIT || s->vc_width || !flags_fit) {
     if (s->thomas == FMS_THOMAS_SERIAL && !s->d_cA &&
         (dalloc(&s->d_cA, (size_t)s->N) || dalloc(&s->d_dA, (size_t)s->N)))
       return FMS_ERR_HIP;
@@ -691,8 +772,17 @@ int run(FmsSolver *s, const double *h_steps, int K, int n0D, bool fused_only) {
   // fused: the kernel reads step s+1's record for the first half of step s+1;
   // a launch covers steps [k0, k0+kc) and then finishes the last step itself
   int rc;
-  if ((rc = upload_steps(s, h_steps, K))) return rc;
-  const int chunk = s->tune_chunk;
+  if ((rc = upload_steps(s, h_steps, K, false))) return rc;
+  int chunk = s->tune_chunk;
+  if constexpr (chunked_model() && fms::is_fma<E>::value) {
+    // the flags of a launch: allocated, or as many steps as the fixed scratch holds
+    chunk = std::min({chunk, K, std::max(1, (1 << 29) / n0D)});
+    if (!s->noalloc) {
+      if (ensure_flag_bytes(s, fibre_flag_bytes(s, chunk, n0D))) return FMS_ERR_HIP;
+    } else {
+      while (chunk > 1 && fibre_flag_bytes(s, chunk, n0D) > s->flags_cap) chunk = (chunk + 1) / 2;
+    }
+  }
   for (int k0 = 0; k0 < K; k0 += chunk) {
     const int kc = std::min(chunk, K - k0);
     if ((rc = launch_fused<G, E>(s, s->d_steps + 4 * (size_t)k0, kc, n0D))) return rc;
@@ -705,7 +795,7 @@ int run(FmsSolver *s, const double *h_steps, int K, int n0D, bool fused_only) {
 // multiply-add forms; the serial solve's runs give the oracle's bits.
 template <class Fn> int with_exp(FmsSolver *s, Fn fn) {
   const bool approx = s->exp_mode == FMS_EXP_APPROXIMATE;
-  if constexpr (Model::NS <= 8) {
+  if constexpr (chunked_model()) {
     if (s->thomas == FMS_THOMAS_PARTITIONED) return approx ? fn(fms::ExpApproxFma{}) : fn(fms::ExpLibmFma{});
   }
   return approx ? fn(fms::ExpApprox{}) : fn(fms::ExpLibm{});
@@ -1191,13 +1281,16 @@ int fms_advance_schedule_noalloc(FmsSolver *s, const double *steps, int n_steps,
                                      "call fms_advance_schedule once first");
   double *keep_steps = s->d_steps;
   unsigned char *keep_flags = s->d_flags;
-  const int keep_steps_cap = s->steps_cap, keep_flags_cap = s->flags_cap, keep_graph = s->tune_graph;
+  const int keep_steps_cap = s->steps_cap, keep_graph = s->tune_graph;
+  const size_t keep_flags_cap = s->flags_cap;
   s->d_steps = reinterpret_cast<double *>(base);
   s->steps_cap = (int)(table_bytes / sizeof(double));
   s->d_flags = base + table_bytes;
-  s->flags_cap = (int)flag_bytes;
+  s->flags_cap = NOALLOC_SCRATCH_BYTES - table_bytes;
   s->tune_graph = 0;   // a graph capture would allocate: eager launches
+  s->noalloc = true;
   const int rc = dispatch(s, steps, n_steps, n0D);
+  s->noalloc = false;
   s->d_steps = keep_steps;
   s->d_flags = keep_flags;
   s->steps_cap = keep_steps_cap;
@@ -1577,7 +1670,8 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
     if (whole && s->tape_cap < (long long)K * (long long)step_len)
       return fail(FMS_ERR_STATE, "the adjoint forward's tape is gone; run fms_adjoint_forward again");
     if (!whole && (rc = ensure(&s->d_tape, s->tape_cap, 2 * (long long)tape_len))) return rc;
-    if ((rc = upload_steps(s, s->adj_steps.data(), K))) return rc;
+    if ((rc = upload_steps(s, s->adj_steps.data(), K, false))) return rc;
+    if (!whole && ensure_flag_bytes(s, fibre_flag_bytes(s, std::min(L, K), n0D))) return FMS_ERR_HIP;
     if (!whole) {
       if (!s->stream2 && hipStreamCreateWithFlags(&s->stream2, hipStreamNonBlocking) != hipSuccess)
         return fail(FMS_ERR_HIP, "hipStreamCreate failed");
@@ -1670,7 +1764,8 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
 }
 
 int adjoint_backward(FmsSolver *s, const double *d_dtraces) {
-  return with_exp(s, [&](auto e) { return adjoint_backward_core<decltype(e)>(s, d_dtraces); });
+  return s->exp_mode == FMS_EXP_APPROXIMATE ? adjoint_backward_core<fms::ExpApproxFma>(s, d_dtraces)
+                                            : adjoint_backward_core<fms::ExpLibmFma>(s, d_dtraces);
 }
 
 // forward over all segments, checkpointing; traces go to device memory d_traces
@@ -1711,14 +1806,14 @@ int adjoint_forward(FmsSolver *s, const double *steps, int n_steps, int n0D, int
     s->d_tape = nullptr;
     s->tape_cap = 0;
   }
-  if (ensure_flags(s, n0D)) return FMS_ERR_HIP;
-  if ((rc = upload_steps(s, steps, K))) return rc;
+  if ((rc = upload_steps(s, steps, K, false))) return rc;
   s->adj_steps.assign(steps, steps + 4 * (size_t)K);
   s->adj_n0D = n0D;
   s->adj_interval = Kc;
   // with the whole tape nothing ties a launch to a segment: the solver's
   // steps per fused launch
   const int len = whole ? s->tune_chunk : Kc;
+  if (ensure_flag_bytes(s, fibre_flag_bytes(s, std::min(len, K), n0D))) return FMS_ERR_HIP;
   for (int seg = 0; seg * (long long)len < K; seg++) {
     const int k0 = seg * len, kc = std::min(len, K - k0);
     if (!whole && (rc = copy_state(s, s->d_ckpt + (size_t)seg * ckpt_doubles(s), true))) return rc;

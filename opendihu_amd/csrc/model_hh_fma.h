@@ -38,7 +38,12 @@ FMS_HD double pow1024(double b) {
   return b;
 }
 
-template <class E> FMS_HD HHExps hh_exps(double V) {
+// the bases 1 + x/1024 of the approximate exponentials, in HHExps's order
+struct HHBases {
+  double m, n, bh, bm, ah, bn;
+};
+
+template <class E> FMS_HD HHExps hh_exps(double V, HHBases *bases = nullptr) {
   HHExps e;
   const double v75 = V + 75.0;
   if constexpr (std::is_base_of<ExpApprox, E>::value) {
@@ -48,9 +53,13 @@ template <class E> FMS_HD HHExps hh_exps(double V) {
     e.em = pow1024(bm);
     e.en = pow1024(bn);
     e.ebh = pow1024(bh);
-    e.ebm = pow1024(__builtin_fma(v75, -1.0 / 18432, 1.0));
-    e.eah = pow1024(__builtin_fma(V, -1.0 / 20480, 1.0 - 3.75 / 1024));
-    e.ebn = pow1024(__builtin_fma(V, 1.0 / 81920, 1.0 + 0.9375 / 1024));
+    const double bbm = __builtin_fma(v75, -1.0 / 18432, 1.0);
+    const double bah = __builtin_fma(V, -1.0 / 20480, 1.0 - 3.75 / 1024);
+    const double bbn = __builtin_fma(V, 1.0 / 81920, 1.0 + 0.9375 / 1024);
+    e.ebm = pow1024(bbm);
+    e.eah = pow1024(bah);
+    e.ebn = pow1024(bbn);
+    if (bases) *bases = HHBases{bm, bn, bh, bbm, bah, bbn};
     e.xm = __builtin_fma(bm, 1024.0, -1024.0);
     e.xn01 = __builtin_fma(bn, 102.4, -102.4);
   } else {
@@ -65,6 +74,24 @@ template <class E> FMS_HD HHExps hh_exps(double V) {
     e.ebn = E::exp(v75 * 0.0125);
   }
   return e;
+}
+
+// 1/base of all six from one reciprocal
+FMS_HD HHBases hh_inverse_bases(const HHBases &b) {
+  const double p2 = b.m * b.n, p3 = p2 * b.bh, p4 = p3 * b.bm, p5 = p4 * b.ah;
+  HHBases r;
+  double q = recip_nr(p5 * b.bn);
+  r.bn = q * p5;
+  q *= b.bn;
+  r.ah = q * p4;
+  q *= b.ah;
+  r.bm = q * p3;
+  q *= b.bm;
+  r.bh = q * p2;
+  q *= b.bh;
+  r.n = q * b.m;
+  r.m = q * b.n;
+  return r;
 }
 
 // 1/(em - 1), 1/(en - 1) and 1/(ebh + 1) from one reciprocal
