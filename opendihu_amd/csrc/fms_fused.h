@@ -7,8 +7,11 @@
 //  * The second reaction half of step s and the first half of step s+1 run in
 //    one pass over the nodes, so each split step reads and writes every gate
 //    once and Vm never touches HBM between launches.
-//  * Diffusion is the partitioned LDS solve (lds_thomas_part) or, for bit-exact
-//    runs, the reference's serial recurrence executed by thread 0 in LDS.
+//  * Diffusion is the partitioned LDS solve (lds_thomas_part, large models) or, for
+//    bit-exact runs, the reference's serial recurrence executed by thread 0 in LDS.
+//    Small models take this kernel for the serial solve only (k_fibre in fms_fibre.h
+//    runs their partitioned one) and keep the matrix factored between steps: 1024
+//    fibres of 101-301 nodes, 200 steps, 30.7 -> 6.2 ms.
 //  * The stimulation state machine of the fibre runs on thread 0 in time order
 //    and hands the per-Heun-step flags to the workgroup through LDS.
 // Uneven fibre lengths: the host orders fibres longest first (LPT) so the
@@ -155,8 +158,8 @@ __global__ __launch_bounds__(T) void k_fused(DevFibers fb, DevStim st, double *_
   const int off = fb.fiber_off[f];
   const int n = fb.fiber_off[f + 1] - off;
   const double pf = fb.prefactor[f];
-  double *red = sh;   // block interfaces of the partitioned solve (pcr_lds_doubles), or the serial solve's cA/dA (16*T doubles)
-  double *lv = sh + (serial ? 16 * T : pcr_lds_doubles<T>());   // n doubles: Vm
+  double *red = sh;   // block interfaces of the partitioned solve, or the serial solve's rows
+  double *lv = sh + (M::NS <= 8 ? serial_lds_doubles(n) : serial ? 16 * T : pcr_lds_doubles<T>());   // n doubles: Vm
   double *h = lv + n;   // n - 1 element lengths, staged once for all the launch's solves
   unsigned char *sflags = (unsigned char *)(h + n);   // 2*n0D flags
 
@@ -251,6 +254,7 @@ __global__ __launch_bounds__(T) void k_fused(DevFibers fb, DevStim st, double *_
   }
   __syncthreads();
 
+  double serial_dt = __builtin_nan("");   // of the factored serial solve: none yet
   for (int s = 0; s < K; s++) {
     const double *st_s = steps + 4 * s;
     const double t_mid = st_s[0] + 0.5 * st_s[1];
@@ -258,10 +262,16 @@ __global__ __launch_bounds__(T) void k_fused(DevFibers fb, DevStim st, double *_
     const bool more = s + 1 < K;
 
     // diffusion (one solve per split step, as the reference)
-    if (M::NS <= 8 || serial) {   // small models: k_fibre takes the partitioned runs
+    if constexpr (M::NS <= 8) {   // k_fibre takes these models' partitioned runs
+      if (dt1 != serial_dt) {
+        serial_factor(red, n, lv, h, pf, dt1, ie != 0, tid, T);
+        serial_dt = dt1;
+      }
+      serial_solve(red, n, lv, h, pf, dt1, ie != 0, tid, T);
+    } else if (serial) {
       if (tid == 0) thomas_serial_fiber(lv, n, h, pf, dt1, ie != 0, red, red + n);
       __syncthreads();
-    } else if constexpr (M::NS > 8) {
+    } else {
       lds_thomas_part<T, MMAX>(lv, n, h, pf, dt1, ie != 0, red, tid);
     }
 

@@ -478,9 +478,8 @@ int launch_thomas(FmsSolver *s, int q) {
     }
   }
   if (s->thomas == FMS_THOMAS_SERIAL) {
-    const int threads = 64;
-    FMS_LAUNCH(s, fms::k_thomas_serial, dim3((s->F + threads - 1) / threads), dim3(threads), 0,
-               s->fibers(), s->d_vm, s->d_cA, s->d_dA, step_ref(s, q), ie);
+    FMS_LAUNCH(s, fms::k_thomas_serial, dim3(s->F), dim3(64), 0, s->fibers(), s->d_vm, s->d_cA, s->d_dA,
+               step_ref(s, q), ie);
   } else {
     // rows per chunk: at most ceil(nmax / 256) (>= 3 for fibres under 512 nodes);
     // the smallest register array that holds them
@@ -651,7 +650,9 @@ template <class G, class E, int T, int NPT, int MMAX>
 int launch_fused_npt(FmsSolver *s, const double *d_steps, int K, int n0D, const fms::DevTrace &tr) {
   KernelTimer timer(s, FMS_KERNEL_FUSED);
   const fms::DevSpikes spk = dev_spikes(s);
-  const int red = s->thomas == FMS_THOMAS_SERIAL ? 16 * T : fms::pcr_lds_doubles<T>();
+  const int red = chunked_model()                   ? fms::serial_lds_doubles(s->nmax)
+                  : s->thomas == FMS_THOMAS_SERIAL ? 16 * T
+                                                   : fms::pcr_lds_doubles<T>();
   const size_t lds = (size_t)(red + 2 * s->nmax) * sizeof(double) + 2 * (size_t)n0D + 16;
   FMS_LAUNCH(s, (fms::k_fused<Model, G, E, T, MMAX, NPT>), dim3(s->F), dim3(T), lds, s->fibers(), s->stim(),
              s->d_vm, (G *)s->d_gates, d_steps, K, n0D, s->vstim, s->scheme == FMS_IMPLICIT_EULER ? 1 : 0,
