@@ -45,7 +45,7 @@ HIP_FLAGS = [
 # scheduler, which is faster for them (occupancy matters there).
 LARGE_MODEL_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 LARGE_MODEL_STATES = 8
-SMALL_MODEL_PARTS = 6   # FMS_PART values of fms_parts.hip
+SMALL_MODEL_PARTS = 8   # FMS_PART values of fms_parts.hip
 
 HH_LIBRARY = "libfms_hodgkin_huxley_1952.so"
 

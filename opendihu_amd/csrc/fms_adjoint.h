@@ -17,30 +17,12 @@
 // the approximate exponential E(x) = (1 + x/1024)^1024, E'(x) = E(x)/(1 + x/1024).
 #pragma once
 
-#include "fms_fused.h"
-#include "model_hh.h"
+#include "fms_fibre.h"
 
 namespace fms {
 
-// a / b for the derivative terms of the linearisation (never for a rate, whose
-// bits must equal the forward's): the device reciprocal refined by one Newton
-// step (which squares its relative error), then one multiply; four instructions
-// instead of the eight of the correctly rounded sequence. The derivatives need
-// no correct rounding: the gradient's agreement with the dense adjoint (1e-9)
-// and with central differences is what the tests hold it to.
-FMS_HD double deriv_div(double a, double b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const double r0 = __builtin_amdgcn_rcp(b);
-  const double r1 = __builtin_fma(r0, __builtin_fma(-b, r0, 1.0), r0);
-  return a * r1;
-#else
-  return a / b;
-#endif
-}
-
 template <class E> struct ExpDeriv;
 template <> struct ExpDeriv<ExpApprox> {
-  static FMS_HD FD d(FD x, FD ex) { return FD(deriv_div(ex.v, (FD(1.0) + x * FD(1.0 / 1024)).v)); }
   // power-series coefficients of E(x) - 1 = sum_k c_k x^k, c_k = binom(1024, k) / 1024^k
   static FMS_HD constexpr double c(int k) {
     double v = 1.0;
@@ -49,7 +31,6 @@ template <> struct ExpDeriv<ExpApprox> {
   }
 };
 template <> struct ExpDeriv<ExpLibm> {
-  static FMS_HD FD d(FD x, FD ex) { (void)x; return ex; }
   static FMS_HD constexpr double c(int k) {   // 1 / k!
     double v = 1.0;
     for (int j = 2; j <= k; j++) v /= j;
@@ -105,97 +86,73 @@ __device__ __forceinline__ double du_near_zero(double x) {
 
 __device__ __forceinline__ bool near_removable(double x) { return x < 0.05 && x > -0.05; }
 
-// Linearisation of the HH right-hand side at y: the rates r(y), computed with
-// the operations of ModelHH::rhs in its order (so y* = y + dt r(y) has the
-// forward's bits), and the partial derivatives that J(y)^T w and
-// f_theta(y)^T w need, from the same exponentials.
+// Linearisation of the HH right-hand side at y: the rates r(y), in the operations
+// of hh_rates_fused (so y* = y + dt r(y) has the forward's bits), and the partial
+// derivatives that J(y)^T w and f_theta(y)^T w need, from the same exponentials.
+// dE/dV = slope E / base: the six bases share one reciprocal. About 190
+// instructions instead of the 340 of an evaluation with a division per quotient
+// and without fused multiply-adds.
 struct HHLin {
   double r[4];
   double f0V, f0m, f0h, f0n;       // d f0 / d(V, m, h, n)
   double f1V, f1m, f2V, f2h, f3V, f3n;
   double gna, gk, gl;              // d f0 / d(g_Na, g_K, g_L)
   FMS_HD void jt(const double *w, double *out) const {
-    out[0] = w[0] * f0V + w[1] * f1V + w[2] * f2V + w[3] * f3V;
-    out[1] = w[0] * f0m + w[1] * f1m;
-    out[2] = w[0] * f0h + w[2] * f2h;
-    out[3] = w[0] * f0n + w[3] * f3n;
-  }
-  FMS_HD void gp(const double *w, double *out) const {
-    out[0] = w[0] * gna;
-    out[1] = w[0] * gk;
-    out[2] = w[0] * gl;
+    out[0] = __builtin_fma(w[0], f0V, __builtin_fma(w[1], f1V, __builtin_fma(w[2], f2V, w[3] * f3V)));
+    out[1] = __builtin_fma(w[0], f0m, w[1] * f1m);
+    out[2] = __builtin_fma(w[0], f0h, w[2] * f2h);
+    out[3] = __builtin_fma(w[0], f0n, w[3] * f3n);
   }
 };
 
 template <class E>
 __device__ __forceinline__ HHLin hh_linearize(const double *y, const double *p) {
-  // FD arithmetic (the forward's division), so r(y) has the forward's bits
   HHLin L;
-  const FD V = y[0], m = y[1], h = y[2], n = y[3];
-  const FD i_stim = p[0], g_na = p[1], g_k = p[2], g_l = p[3];
-  const FD constant0 = FD(-75), constant1 = FD(1);
-  const FD constant6 = constant0 + FD(115.000), constant7 = constant0 - FD(12.0000);
-  const FD constant8 = constant0 + FD(10.6130);
-  // rates, in ModelHH::rhs's operation order
-  const FD em = E::exp(-(V + FD(50.0000)) / FD(10.0000));
-  const FD a1 = (FD(-0.100000) * (V + FD(50.0000))) / (em - FD(1.00000));
-  const FD ebm = E::exp(-(V + FD(75.0000)) / FD(18.0000));
-  const FD a5 = FD(4.00000) * ebm;
-  const FD r1 = a1 * (FD(1.00000) - m) - a5 * m;
-  const FD eah = E::exp(-(V + FD(75.0000)) / FD(20.0000));
-  const FD a2 = FD(0.0700000) * eah;
-  const FD ebh = E::exp(-(V + FD(45.0000)) / FD(10.0000));
-  const FD a6 = FD(1.00000) / (ebh + FD(1.00000));
-  const FD r2 = a2 * (FD(1.00000) - h) - a6 * h;
-  const FD en = E::exp(-(V + FD(65.0000)) / FD(10.0000));
-  const FD a3 = (FD(-0.0100000) * (V + FD(65.0000))) / (en - FD(1.00000));
-  const FD ebn = E::exp((V + FD(75.0000)) / FD(80.0000));
-  const FD a7 = FD(0.125000) * ebn;
-  const FD r3 = a3 * (FD(1.00000) - n) - a7 * n;
-  const FD m3 = pow3(m), n4 = pow4(n);
-  const FD a0 = g_na * m3 * h * (V - constant6);
-  const FD a4 = g_k * n4 * (V - constant7);
-  const FD a8 = g_l * (V - constant8);
-  const FD r0 = -(-i_stim + a0 + a4 + a8) / constant1;
-  L.r[0] = r0.v; L.r[1] = r1.v; L.r[2] = r2.v; L.r[3] = r3.v;
-  // derivatives (E'(x) of the exponential actually used)
-  const FD xm = -(V + FD(50.0000)) / FD(10.0000), xbm = -(V + FD(75.0000)) / FD(18.0000);
-  const FD xah = -(V + FD(75.0000)) / FD(20.0000), xbh = -(V + FD(45.0000)) / FD(10.0000);
-  const FD xn = -(V + FD(65.0000)) / FD(10.0000), xbn = (V + FD(75.0000)) / FD(80.0000);
-  // d alpha_m / dV = -0.1 u'(xm), d alpha_n / dV = -0.01 u'(xn) (u above): the
-  // quotient rule u' = (E - 1 - x E') / (E - 1)^2, and the series within
-  // |x| < 0.05 of a singular voltage
-  const FD den_m = em - FD(1.0);
-  double dum = deriv_div((den_m - xm * ExpDeriv<E>::d(xm, em)).v, (den_m * den_m).v);
-  const FD dbm = FD(4.0) * ExpDeriv<E>::d(xbm, ebm) * FD(-1.0 / 18.0);
-  const FD dah = FD(0.07) * ExpDeriv<E>::d(xah, eah) * FD(-1.0 / 20.0);
-  const FD dbh = FD(deriv_div((-(ExpDeriv<E>::d(xbh, ebh) * FD(-0.1))).v, ((ebh + FD(1.0)) * (ebh + FD(1.0))).v));
-  const FD den_n = en - FD(1.0);
-  double dun = deriv_div((den_n - xn * ExpDeriv<E>::d(xn, en)).v, (den_n * den_n).v);
-  // a lane is near at most one of the two singular voltages (1.5 apart in x).
-  // The polynomial is evaluated on every lane and selected: a branch here (even
-  // a wave-uniform one) splits the unrolled per-node code into blocks that the
-  // scheduler cannot interleave, which measured 1.9x slower at one wave per SIMD.
-  const bool near_m = near_removable(xm.v), near_n = near_removable(xn.v);
-  const double dus = du_near_zero<E>(near_m ? xm.v : xn.v);
-  dum = near_m ? dus : dum;
-  dun = near_n ? dus : dun;
-  const FD dam = FD(-0.1 * dum), dan = FD(-0.01 * dun);
-  const FD dbn = FD(0.125) * ExpDeriv<E>::d(xbn, ebn) * FD(1.0 / 80.0);
-  const FD m2 = m * m, n3 = n * n * n;
-  L.f0V = (-(g_na * m3 * h + g_k * n4 + g_l)).v;
-  L.f0m = (-(g_na * FD(3.0) * m2 * h * (V - constant6))).v;
-  L.f0h = (-(g_na * m3 * (V - constant6))).v;
-  L.f0n = (-(g_k * FD(4.0) * n3 * (V - constant7))).v;
-  L.f1V = (dam * (FD(1.0) - m) - dbm * m).v;
-  L.f1m = (-a1 - a5).v;
-  L.f2V = (dah * (FD(1.0) - h) - dbh * h).v;
-  L.f2h = (-a2 - a6).v;
-  L.f3V = (dan * (FD(1.0) - n) - dbn * n).v;
-  L.f3n = (-a3 - a7).v;
-  L.gna = (-m3 * h * (V - constant6)).v;
-  L.gk = (-n4 * (V - constant7)).v;
-  L.gl = (-(V - constant8)).v;
+  const double V = y[0], m = y[1], h = y[2], n = y[3];
+  HHBases b;
+  const HHExps e = hh_exps<E>(V, &b);
+  double im, in, ih;
+  hh_inverses(e, im, in, ih);
+  const double am = e.xm * im, an = e.xn01 * in;
+  const double ah = 0.07 * e.eah, bm = 4.0 * e.ebm, bn = 0.125 * e.ebn;
+  const double sm = __builtin_fma(4.0, e.ebm, am), sh = ah + ih, sn = __builtin_fma(0.125, e.ebn, an);
+  L.r[1] = __builtin_fma(-sm, m, am);
+  L.r[2] = __builtin_fma(-sh, h, ah);
+  L.r[3] = __builtin_fma(-sn, n, an);
+  const double m2 = m * m, m3 = m2 * m, m3h = m3 * h, n2 = n * n, n4 = n2 * n2;
+  const double gm3h = p[1] * m3h, gn4 = p[2] * n4;
+  const double vna = V - 40.0, vk = V + 87.0, vl = V + (75.0 - 10.6130);
+  L.r[0] = __builtin_fma(-gm3h, vna, __builtin_fma(-gn4, vk, -(p[3] * vl))) + p[0];
+  // E'(x) of the exponential used, divided by it: 1/base (approximate), 1 (exact)
+  HHBases ib{1.0, 1.0, 1.0, 1.0, 1.0, 1.0};
+  if constexpr (std::is_base_of<ExpApprox, E>::value) ib = hh_inverse_bases(b);
+  // alpha_m = u(xm), alpha_n = u(xn) / 10 (u above): u' = (1 - u E') / (E - 1) by the
+  // quotient rule, and the series within |x| < 0.05 of a singular voltage. A lane is
+  // near at most one of the two singular voltages (1.5 apart in x). The polynomial is
+  // evaluated on every lane and selected: a branch would split the nodes' code into
+  // blocks that the scheduler cannot interleave.
+  const double xn = 10.0 * e.xn01;
+  const bool near_m = near_removable(e.xm), near_n = near_removable(xn);
+  const double dus = du_near_zero<E>(near_m ? e.xm : xn);
+  const double dum = near_m ? dus : im * __builtin_fma(-am, e.em * ib.m, 1.0);
+  const double dun = near_n ? dus : in * __builtin_fma(-10.0 * an, e.en * ib.n, 1.0);
+  const double dam = -0.1 * dum, dan = -0.01 * dun;
+  const double dbm = bm * ib.bm * (-1.0 / 18.0), dah = ah * ib.ah * (-1.0 / 20.0);
+  const double dbh = ih * ih * (e.ebh * ib.bh) * 0.1, dbn = bn * ib.bn * (1.0 / 80.0);
+  L.f0V = -(gm3h + gn4 + p[3]);
+  const double gv = -p[1] * vna;
+  L.f0m = 3.0 * m2 * h * gv;
+  L.f0h = m3 * gv;
+  L.f0n = -4.0 * (p[2] * vk) * (n2 * n);
+  L.f1V = __builtin_fma(-(dam + dbm), m, dam);
+  L.f1m = -sm;
+  L.f2V = __builtin_fma(-(dah + dbh), h, dah);
+  L.f2h = -sh;
+  L.f3V = __builtin_fma(-(dan + dbn), n, dan);
+  L.f3n = -sn;
+  L.gna = -(m3h * vna);
+  L.gk = -(n4 * vk);
+  L.gl = -vl;
   return L;
 }
 
@@ -203,217 +160,269 @@ __device__ __forceinline__ HHLin hh_linearize(const double *y, const double *p) 
 // lam[4] in: adjoint of the output, out: adjoint of y; gacc[3] += parameter gradient
 template <class E>
 __device__ __forceinline__ void hh_heun_step_reverse(const double *y, const double *p, double dt, double *lam, double *gacc) {
+  const double hdt = 0.5 * dt;
   const HHLin Ly = hh_linearize<E>(y, p);
   double ys[4];
-  for (int k = 0; k < 4; k++) ys[k] = y[k] + dt * Ly.r[k];
-  const HHLin Ls = hh_linearize<E>(ys, p);
-  double mu[4], gs[3], nu[4], jy[4], g3[3];
-  Ls.jt(lam, mu);
-  Ls.gp(lam, gs);
-  for (int k = 0; k < 4; k++) nu[k] = lam[k] + dt * mu[k];
+#pragma unroll
+  for (int k = 0; k < 4; k++) ys[k] = __builtin_fma(dt, Ly.r[k], y[k]);
+  double mu[4], nu[4], jy[4], gs[3];
+  {
+    const HHLin Ls = hh_linearize<E>(ys, p);
+    Ls.jt(lam, mu);
+    gs[0] = lam[0] * Ls.gna;
+    gs[1] = lam[0] * Ls.gk;
+    gs[2] = lam[0] * Ls.gl;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; k++) nu[k] = __builtin_fma(dt, mu[k], lam[k]);
   Ly.jt(nu, jy);
-  Ly.gp(nu, g3);
-  for (int k = 0; k < 4; k++) lam[k] = lam[k] + 0.5 * dt * mu[k] + 0.5 * dt * jy[k];
-  for (int k = 0; k < 3; k++) gacc[k] += 0.5 * dt * (g3[k] + gs[k]);
-}
-
-// current-pulse stimulus parameter of one Heun step, as the forward sets it
-// (the pulse is a constant of each Heun step; fms_fused.h fused_node_half).
-// Selects per element, not a store at a run-time index, so pj stays in registers.
-template <class E>
-FMS_HD void stim_params(const DevStim &st, int f, bool inset, const double *p, double t, double *pj) {
-  const bool pulse = st.mode == 2 && current_on(st, f, t) && inset;
 #pragma unroll
-  for (int k = 0; k < 4; k++) pj[k] = pulse && k == st.stim_param ? st.amplitude[f] : p[k];
+  for (int k = 0; k < 4; k++) lam[k] = __builtin_fma(hdt, mu[k] + jy[k], lam[k]);
+  gacc[0] = __builtin_fma(hdt, __builtin_fma(nu[0], Ly.gna, gs[0]), gacc[0]);
+  gacc[1] = __builtin_fma(hdt, __builtin_fma(nu[0], Ly.gk, gs[1]), gacc[1]);
+  gacc[2] = __builtin_fma(hdt, __builtin_fma(nu[0], Ly.gl, gs[2]), gacc[2]);
 }
 
-// reverse of one reaction half of a thread's NPT nodes, each from its state
-// y0[q] at t0: l[q] in: adjoint of the half's output, out: adjoint of y0[q];
-// g[q] += dL/d(gNa, gK, gL). Heun step j is reversed from its recomputed input
-// with the stimulus parameter of that step (a per-lane select), so all lanes
-// take the same path. The node loop is the innermost one: the NPT nodes'
-// independent linearisations then share one basic block, which the scheduler
-// interleaves (a node loop around the run-time loop over the Heun steps gives
-// one block per node and a single dependency chain at a time).
-template <class E, int NPT>
-__device__ __forceinline__ void reverse_half(const DevStim &st, int f, const bool *inset, const double (*y0)[4],
-                                             const double *p, double t0, double dt, int n0D, double (*l)[4],
-                                             double (*g)[3]) {
+// current pulses as the reverse sweep sees them
+struct AdjStim {
+  int on;       // pulses are set
+  int param;    // the stimulus parameter
+  const double *onset, *duration, *amplitude;   // [F]
+};
+
+// reverse of one reaction half of a node from its state y0 at t0: l in: adjoint of
+// the half's output, out: adjoint of y0; g += dL/d(gNa, gK, gL). Heun step j is
+// reversed from its recomputed input with the stimulus parameter of that step
+// (params(t, p)).
+template <class E, class Params>
+__device__ __forceinline__ void reverse_half(Params &&params, const double *y0, double t0, double dt, int n0D,
+                                             double *l, double *g) {
+#pragma unroll 1
   for (int j = n0D - 1; j >= 0; j--) {
-    double y[NPT][4];
-#pragma unroll
-    for (int q = 0; q < NPT; q++)
-#pragma unroll
-      for (int k = 0; k < 4; k++) y[q][k] = y0[q][k];
+    double y[4] = {y0[0], y0[1], y0[2], y0[3]}, pj[4];
+#pragma unroll 1
     for (int jj = 0; jj < j; jj++) {
-#pragma unroll
-      for (int q = 0; q < NPT; q++) {
-        double pj[4];
-        stim_params<E>(st, f, inset[q], p, t0 + jj * dt, pj);
-        heun_node<ModelHH, double, E, false>(y[q][0], y[q] + 1, pj, t0 + jj * dt, dt, false, 0.0);
-      }
+      params(t0 + jj * dt, pj);
+      heun_node<ModelHH, double, E, false>(y[0], y + 1, pj, t0 + jj * dt, dt, false, 0.0);
     }
-#pragma unroll
-    for (int q = 0; q < NPT; q++) {
-      double pj[4];
-      stim_params<E>(st, f, inset[q], p, t0 + j * dt, pj);
-      hh_heun_step_reverse<E>(y[q], pj, dt, l[q], g[q]);
-    }
+    params(t0 + j * dt, pj);
+    hh_heun_step_reverse<E>(y, pj, dt, l, g);
   }
 }
 
-// Reverse of kc split steps of one segment, one workgroup per fibre, steps
-// s = kc-1 .. 0 (rows of `steps`, 4 doubles each). Per step: the sensors'
-// dL/dV, reverse of half 2 from y^b = (V^b, gates after half 1), reverse
-// diffusion w = A^{-1} lambda_V, lambda_V = B w (A, B symmetric),
-// pf_bar += w^T (dB/dpf V^a - dA/dpf V^b), reverse of half 1 from y0. lambda and
-// the per-node parameter gradients stay in registers for the whole segment.
-// Tape: [kc][9][N] = y0 (4), y after half 1 (V^a and the gates, 4), V^b.
-template <class E, int T, int NPT, int MMAX>
-__global__ __launch_bounds__(T) void k_adj_fused(DevFibers fb, DevStim st, const double *__restrict__ tape,
-                                                 const double *__restrict__ steps, int kc, int n0D, int ie,
-                                                 const int *__restrict__ sensor_slot,
-                                                 const double *__restrict__ dtrace, int n_sensors, double *lam,
-                                                 double *gacc, double *pf_bar, int raise_priority) {
+// What one launch of the reverse sweep needs: kc split steps of one segment, steps
+// s = kc-1 .. 0 (rows of `steps`). Tape: [kc][9][N] = y0 (4), y after half 1 (V^a and
+// the gates, 4), V^b. lam: [4][N]; acc: [4][F * T], each thread's sums of dL/d(gNa, gK,
+// gL) and of the prefactor's element terms.
+struct AdjArgs {
+  DevFibers fb;
+  AdjStim st;
+  const double *tape, *steps;
+  int kc, n0D, ie;
+  const int *sensor_slot;
+  const double *dtrace;
+  int n_sensors;
+  double *lam, *acc;
+  int raise_priority;
+};
+
+// Per step: the sensors' dL/dV, reverse of half 2 from y^b = (V^b, gates after half
+// 1), reverse diffusion, reverse of half 1 from y0. A w = lambda_V is solved with the
+// factored chunks of the forward (fms_chunk.h: A' x = lambda_V, w = -x), and B = A - K
+// gives B w = lambda_V + K x, a difference of element fluxes; the same fluxes give
+// the prefactor gradient w^T (dB/dpf V^a - dA/dpf V^b) = -theta sum_e (x_{e+1} - x_e)
+// (v_{e+1} - v_e) / h_e with v = V^b, theta = 1 (IE) or v = V^a + V^b, theta = 1/2 (CN).
+// lambda, and the sums of each thread, stay in registers for the whole segment; sums
+// over threads are taken once after the last segment (k_adj_reduce), so the gradient
+// does not depend on the segmentation.
+template <class E, int T, int C>
+__device__ __forceinline__ void adj_steps(const AdjArgs &a, int f, int off, int n, double *sh) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const long long N = a.fb.n_total, FT = (long long)a.fb.n_fibers * T;
+  const double pf = a.fb.prefactor[f];
+  const ChunkLds<T, C> lds{sh, tid};
+  const int lo = tid * C;
+  const bool busy = wave * 64 * C < n;
+  const bool ie = a.ie != 0;
+  double p[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) p[k] = a.fb.params[(long long)f * 4 + k];
+  const double onset = a.st.on ? a.st.onset[f] - 1e-13 : 0.0;
+  const double end = a.st.on ? a.st.onset[f] + a.st.duration[f] - 1e-13 : 0.0;
+  const double amp = a.st.on ? a.st.amplitude[f] : 0.0;
+  double l[C][4], acc[4];
+  int slot[C];
+  unsigned inset = 0;
+  {
+    const int sb = a.fb.stim_begin[f], se = a.fb.stim_end[f];
+#pragma unroll
+    for (int q = 0; q < C; q++) {
+      // threads past the fibre's end shadow its last node with a zero adjoint
+      const bool valid = lo + q < n;
+      const int i = off + (valid ? lo + q : n - 1);
+#pragma unroll
+      for (int k = 0; k < 4; k++) l[q][k] = valid ? a.lam[k * N + i] : 0.0;
+      slot[q] = valid ? a.sensor_slot[i] : -1;
+      inset |= (lo + q >= sb && lo + q < se ? 1u : 0u) << q;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) acc[k] = a.acc[k * FT + (long long)f * T + tid];
+  }
+  // the element between the previous wave's last node and this wave's first
+  const double ihl = lane == 0 && wave > 0 && lo < n ? recip_nr(a.fb.elem_len[off - f + lo - 1]) : 0.0;
+  // half step hs: the second half of step hs / 2 and its diffusion (odd), or its
+  // first half. One node at a time (its two linearisations hold about 100
+  // registers; two waves per SIMD hide their chains), the next node's tape entries
+  // in flight meanwhile, over the end of a half and the solve too.
+  struct NodeTape {
+    double y[4], va, dl;   // the state the half starts from; V^a; the sensor's dL/dV
+  };
+  double v[C];   // the diffusion's Vm
+  auto load = [&](int hs, int q) {
+    NodeTape in;
+    const int s = hs >> 1;
+    const double *tp = a.tape + (long long)s * 9 * N + off + (lo + q < n ? lo + q : n - 1);
+    in.va = 0.0;
+    in.dl = 0.0;
+    if (hs & 1) {
+      in.y[0] = tp[8 * N];
+#pragma unroll
+      for (int k = 1; k < 4; k++) in.y[k] = tp[(4 + k) * N];
+      if (!ie) in.va = tp[4 * N];
+      if (slot[q] >= 0) in.dl = a.dtrace[((long long)s * a.fb.n_fibers + f) * a.n_sensors + slot[q]];
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; k++) in.y[k] = tp[k * N];
+    }
+    return in;
+  };
+#pragma unroll
+  for (int q = 0; q < C; q++) v[q] = 0.0;
+  int hs = 2 * a.kc - 1;
+  NodeTape next{};
+  if (busy) next = load(hs, 0);
+  while (hs >= 0) {
+    const double dt1 = a.steps[4 * (long long)(hs >> 1) + 3];
+    ChunkFactor<C> fac;
+    chunk_refactor<T, C, true>(fac, n, a.fb.elem_len + (off - f), pf, dt1, ie, lds);
+#pragma unroll 1
+    do {
+      const int s = hs >> 1;
+      const bool half = hs & 1;
+      const double *row = a.steps + 4 * (long long)s;
+      if (busy) {
+        const double t0 = half_start(row, half), dt = row[2];
+        constexpr_for<0, C, 1>([&](auto q_) {
+          constexpr int q = decltype(q_)::value;
+          const NodeTape in = next;
+          if constexpr (q + 1 < C)
+            next = load(hs, q + 1);
+          else if (hs > 0)
+            next = load(hs - 1, 0);
+          if (half) {
+            l[q][0] += in.dl;
+            v[q] = in.va + in.y[0];   // V^b, or V^a + V^b
+          }
+          auto params = [&](double t, double *pj) {
+            // the pulse's window as the forward has it (current_on)
+            const bool on = a.st.on && t >= onset && t < end && ((inset >> q) & 1);
+#pragma unroll
+            for (int k = 0; k < 4; k++) pj[k] = on && k == a.st.param ? amp : p[k];
+          };
+          reverse_half<E>(params, in.y, t0, dt, a.n0D, l[q], acc);
+        });
+      }
+      hs--;
+      if (!half) continue;
+      // A' x = lambda_V; rows past the fibre's end have no coefficients
+      double z[C];
+#pragma unroll
+      for (int q = 0; q < C; q++) z[q] = lo + q < n ? l[q][0] : 0.0;
+      double D = z[0], zlast = 0.0;
+      chunk_interior<C>(fac, z);
+      if constexpr (C > 1) {
+        zlast = z[C - 1];
+        D = __builtin_fma(-fac.o0, z[1], D);
+      }
+      D -= lane_prev(fac.ob * zlast);
+      double X, Xn, Sn, Lp;
+      chunk_separators<T, C>(fac, D, zlast, v[0], 0.0, s & 1, lds, X, Xn, Sn, Lp);
+      constexpr_for<1, C, 1>([&](auto k_) {
+        constexpr int k = decltype(k_)::value;
+        z[k] = __builtin_fma(lds.zr(k), Xn, __builtin_fma(lds.zl(k), X, z[k]));
+      });
+      z[0] = X;
+      // fluxes of x over the thread's elements: lambda_V += K x, prefactor terms
+      double xn = lane_next(X), vn = lane_next(v[0]);
+      if (lane == 63) {
+        xn = Sn;
+        vn = wave + 1 < T / 64 ? lds.iface(s & 1)[4 * (wave + 1)] : 0.0;
+      }
+      double fx[C], pfs = 0.0;
+#pragma unroll
+      for (int q = 0; q < C; q++) {
+        const double ih = q == C - 1 ? fac.kapb : fac.kap[q];
+        fx[q] = ih * ((q == C - 1 ? xn : z[q + 1 < C ? q + 1 : q]) - z[q]);
+        pfs = __builtin_fma(fx[q], (q == C - 1 ? vn : v[q + 1 < C ? q + 1 : q]) - v[q], pfs);
+      }
+      acc[3] -= pfs;
+      // the flux of the element left of the first row: the previous thread's last; at
+      // the start of a wave from the previous wave's last row
+      double fp = lane_prev(fx[C - 1]);
+      if (lane == 0) fp = ihl * (X - Lp);
+#pragma unroll
+      for (int q = 0; q < C; q++) {
+        l[q][0] = __builtin_fma(pf, fx[q] - fp, l[q][0]);
+        fp = fx[q];
+      }
+    } while (hs >= 0 && (!(hs & 1) || a.steps[4 * (long long)(hs >> 1) + 3] == dt1));
+  }
+#pragma unroll
+  for (int q = 0; q < C; q++)
+    if (lo + q < n) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) a.lam[k * N + off + lo + q] = l[q][k];
+    }
+#pragma unroll
+  for (int k = 0; k < 4; k++) a.acc[k * FT + (long long)f * T + tid] = acc[k];
+}
+
+template <class E, int T, int CMAX>
+__global__ __launch_bounds__(T, 2) void k_adj_steps(AdjArgs a) {
   extern __shared__ double sh[];
   // with raise_priority the reverse sweep's waves win issue over the next
   // segment's recompute that runs beside it on the same CUs
-  if (raise_priority) __builtin_amdgcn_s_setprio(2);
+  if (a.raise_priority) __builtin_amdgcn_s_setprio(2);
   const int f = blockIdx.x;
-  const int tid = threadIdx.x;
-  const long long N = fb.n_total;
-  const int off = fb.fiber_off[f];
-  const int n = fb.fiber_off[f + 1] - off;
-  const double pf = fb.prefactor[f];
-  double *red = sh;                          // partitioned solve's block interfaces (pcr_lds_doubles)
-  double *lw = sh + pcr_lds_doubles<T>();    // n: lambda_V, then w
-  double *lv = lw + n;       // n: the diffusion's V (IE: V^b, CN: V^a + V^b), for the neighbours
-  double *h = lv + n;        // n - 1 element lengths, staged once (read after the first step's barrier)
-  for (int i = tid; i < n - 1; i += T) h[i] = fb.elem_len[off - f + i];
-  double p[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) p[k] = fb.params[(long long)f * 4 + k];
-  const int sb = fb.stim_begin[f], se = fb.stim_end[f];
-  double l[NPT][4], g[NPT][3];
-  int slot[NPT];
-  bool inset[NPT];
-  double pfacc = 0;
-  // the fibre's running prefactor gradient, held by thread 0 for the segment:
-  // the same additions in the same order as adding to pf_bar[f] every step
-  double pftotal = tid == 0 ? pf_bar[f] : 0.0;
-  // lanes past the fibre's end shadow its last node: they compute, never store
-#pragma unroll
-  for (int q = 0; q < NPT; q++) {
-    const int i = tid + q * T < n ? tid + q * T : n - 1;
-#pragma unroll
-    for (int k = 0; k < 4; k++) l[q][k] = lam[k * N + off + i];
-#pragma unroll
-    for (int k = 0; k < 3; k++) g[q][k] = gacc[k * N + off + i];
-    slot[q] = sensor_slot[off + i];
-    inset[q] = i >= sb && i < se;
-  }
-  for (int s = kc - 1; s >= 0; s--) {
-    const double *row = steps + 4 * s;
-    const double t = row[0], dts = row[1], dt0 = row[2], dt1 = row[3];
-    // all of the step's tape entries and sensor adjoints are loaded up front
-    // (loading them a step ahead instead measured 1.9x slower: the extra live
-    // registers push the linearisation into AGPRs)
-    const double *tp = tape + (long long)s * 9 * N;
-    double yb[NPT][4], y0[NPT][4], va[NPT], dl[NPT];
-#pragma unroll
-    for (int q = 0; q < NPT; q++) {
-      const long long node = off + (tid + q * T < n ? tid + q * T : n - 1);
-      yb[q][0] = tp[8 * N + node];
-      yb[q][1] = tp[5 * N + node];
-      yb[q][2] = tp[6 * N + node];
-      yb[q][3] = tp[7 * N + node];
-      y0[q][0] = tp[node];
-      y0[q][1] = tp[N + node];
-      y0[q][2] = tp[2 * N + node];
-      y0[q][3] = tp[3 * N + node];
-      va[q] = tp[4 * N + node];
-      dl[q] = dtrace[((long long)s * fb.n_fibers + f) * n_sensors + (slot[q] >= 0 ? slot[q] : 0)];
-    }
-    // sensors, reverse of half 2 from y^b (V after the diffusion, gates after half 1)
-#pragma unroll
-    for (int q = 0; q < NPT; q++) {
-      const bool valid = tid + q * T < n;
-      const int i = valid ? tid + q * T : n - 1;
-      l[q][0] += slot[q] >= 0 ? dl[q] : 0.0;
-      if (valid) lv[i] = ie ? yb[q][0] : va[q] + yb[q][0];
-    }
-    reverse_half<E, NPT>(st, f, inset, yb, p, t + 0.5 * dts, dt0, n0D, l, g);
-#pragma unroll
-    for (int q = 0; q < NPT; q++)
-      if (tid + q * T < n) lw[tid + q * T] = l[q][0];
-    __syncthreads();
-    // reverse diffusion
-    lds_thomas_part<T, MMAX, true>(lw, n, h, pf, dt1, ie != 0, red, tid);
-#pragma unroll
-    for (int q = 0; q < NPT; q++) {
-      const bool valid = tid + q * T < n;
-      const int i = valid ? tid + q * T : n - 1;
-      double a, b, c, d;
-      assemble_row(i, n, lw, h, pf, dt1, ie != 0, a, b, c, d);   // d = (B w)_i
-      const double vi = lv[i];
-      double k1v = 0;
-      if (i > 0) k1v += (lv[i - 1] - vi) / h[i - 1];
-      if (i < n - 1) k1v += (lv[i + 1] - vi) / h[i];
-      pfacc += valid ? lw[i] * (ie ? -k1v : -0.5 * k1v) : 0.0;
-      l[q][0] = d;
-    }
-    // this step's prefactor gradient, summed in a fixed order (butterfly within
-    // each wave, then the waves in order) and added to the fibre's total step by
-    // step, so the result does not depend on the checkpoint segmentation
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) pfacc += __shfl_xor(pfacc, o, 64);
-    if ((tid & 63) == 0) red[tid >> 6] = pfacc;
-    pfacc = 0;
-    __syncthreads();
-    if (tid == 0) {
-      double sum = red[0];
-#pragma unroll
-      for (int q = 1; q < T / 64; q++) sum += red[q];
-      pftotal += sum;
-    }
-    // (every read of lw and lv above precedes that barrier, and the next step
-    // writes red only after the barrier that follows its first loop, so thread
-    // 0's read of red needs no barrier of its own)
-    // reverse of half 1
-    reverse_half<E, NPT>(st, f, inset, y0, p, t, dt0, n0D, l, g);
-  }
-  if (tid == 0) pf_bar[f] = pftotal;
-#pragma unroll
-  for (int q = 0; q < NPT; q++) {
-    const int i = tid + q * T;
-    if (i < n) {
-#pragma unroll
-      for (int k = 0; k < 4; k++) lam[k * N + off + i] = l[q][k];
-#pragma unroll
-      for (int k = 0; k < 3; k++) gacc[k * N + off + i] = g[q][k];
-    }
-  }
+  const int off = a.fb.fiber_off[f];
+  const int n = a.fb.fiber_off[f + 1] - off;
+  with_chunk_rows<CMAX>((n + T - 1) / T,
+                        [&](auto c_) { adj_steps<E, T, decltype(c_)::value>(a, f, off, n, sh); });
 }
 
-// per-fibre sums of the per-node parameter-gradient accumulators
-static __global__ void k_adj_reduce(DevFibers fb, const double *gacc, double *grad) {
+// per-fibre sums of the threads' accumulators [4][F * T], in a fixed order: the
+// conductances' gradients to grad [F][3], the prefactor's (scaled by theta) to
+// pf_bar [F]
+static __global__ __launch_bounds__(256) void k_adj_reduce(int n_fibers, int T, const double *acc, double theta,
+                                                           double *grad, double *pf_bar) {
   const int f = blockIdx.x;
-  const int off = fb.fiber_off[f], n = fb.fiber_off[f + 1] - off;
-  __shared__ double part[3][256];
-  double s0 = 0, s1 = 0, s2 = 0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    s0 += gacc[off + i];
-    s1 += gacc[fb.n_total + off + i];
-    s2 += gacc[2 * fb.n_total + off + i];
-  }
-  part[0][threadIdx.x] = s0;
-  part[1][threadIdx.x] = s1;
-  part[2][threadIdx.x] = s2;
-  __syncthreads();
-  if (threadIdx.x < 3) {
+  const long long FT = (long long)n_fibers * T;
+  __shared__ double part[4][256];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
     double s = 0;
-    for (int q = 0; q < (int)blockDim.x; q++) s += part[threadIdx.x][q];
-    grad[f * 3 + threadIdx.x] = s;
+    for (int i = threadIdx.x; i < T; i += 256) s += acc[k * FT + (long long)f * T + i];
+    part[k][threadIdx.x] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    double s = 0;
+    for (int q = 0; q < 256; q++) s += part[threadIdx.x][q];
+    if (threadIdx.x < 3)
+      grad[f * 3 + threadIdx.x] = s;
+    else
+      pf_bar[f] = theta * s;
   }
 }
 

@@ -333,8 +333,13 @@ __device__ __forceinline__ void chunk_chain(const double *iface, const double *b
     const double L = tmp[4 * w + 2] + tmp[4 * w + 3] * Fn;
     if (w < W - 1 && (w == wave || w == wave - 1)) {
       const double o = bnd[8 * w + BND_O], f = bnd[8 * w + BND_KAP] * (iface[4 * (w + 1)] - iface[4 * w + 2]);
-      ChunkBoundary &b = w == wave ? right : left;
-      b = ChunkBoundary{f - o * Fn, f + o * L, Fn, L};
+      // (selects: a reference to one of the two would put both into the stack frame)
+      const bool r = w == wave;
+      const double rho = f - o * Fn, gamma = f + o * L;
+      right.rho = r ? rho : right.rho;
+      right.S = r ? Fn : right.S;
+      left.gamma = r ? left.gamma : gamma;
+      left.L = r ? left.L : L;
     }
     Fn = tmp[4 * w] + tmp[4 * w + 1] * Fn;
   }

@@ -191,6 +191,35 @@ __device__ __forceinline__ void fibre_heun(double *V, G (*g)[M::NS - 1], const d
   });
 }
 
+// C consecutive doubles of a thread's nodes to the tape, two per store (8-byte
+// aligned: one store per node left each cache line to C partial writes)
+typedef double double2_a8 __attribute__((ext_vector_type(2), aligned(8)));
+template <int C> __device__ __forceinline__ void tape_row(double *dst, int lo, int n, const double *v) {
+  constexpr_for<0, C, 2>([&](auto k_) {
+    constexpr int k = decltype(k_)::value;
+    if constexpr (k + 1 < C) {
+      if (lo + k + 1 < n) {
+        *reinterpret_cast<double2_a8 *>(dst + k) = double2_a8{v[k], v[k + 1]};
+        return;
+      }
+    }
+    if (lo + k < n) dst[k] = v[k];
+  });
+}
+// Vm and the gates
+template <class M, class G, int C>
+__device__ __forceinline__ void tape_state(double *dst, long long N, int lo, int n, const double *V,
+                                           const G (*g)[M::NS - 1]) {
+  tape_row<C>(dst, lo, n, V);
+#pragma unroll
+  for (int q = 0; q < M::NS - 1; q++) {
+    double v[C];
+#pragma unroll
+    for (int k = 0; k < C; k++) v[k] = (double)g[k][q];
+    tape_row<C>(dst + (q + 1) * N, lo, n, v);
+  }
+}
+
 // the fibre's steps with C nodes per thread; TAPE: sensor traces and the adjoint's
 // tape are recorded (either may be absent)
 template <class M, class G, class E, int T, int C, bool TAPE>
@@ -230,6 +259,10 @@ __device__ __forceinline__ void fibre_steps(const DevFibers &fb, const FibreStim
   }
   const bool wave_inset = __builtin_amdgcn_ballot_w64(inset != 0) != 0;
 
+  // the thread's first node in row `slot` of step s's tape
+  auto tape_at = [&](int s, int slot) {
+    return tr.tape + ((long long)s * (2 * M::NS + 1) + slot) * fb.n_total + off + lo;
+  };
   // half step hs: the first reaction half of step hs / 2, or (odd) its diffusion
   // and second reaction half. The outer loop runs once per change of dt.
   int hs = 0;
@@ -246,14 +279,10 @@ __device__ __forceinline__ void fibre_steps(const DevFibers &fb, const FibreStim
       if (half) chunk_diffuse<T, C>(fac, V, s & 1, lds);
       if (TAPE && tr.tape) {
         // half 0: the state before it; half 1: Vm after the diffusion
-#pragma unroll
-        for (int k = 0; k < C; k++)
-          if (lo + k < n) {
-            if (half)
-              tape_store<M::NS>(tr, fb.n_total, s, 2 * M::NS, off + lo + k, V[k], g[k], 1);
-            else
-              tape_store<M::NS>(tr, fb.n_total, s, 0, off + lo + k, V[k], g[k], M::NS);
-          }
+        if (half)
+          tape_row<C>(tape_at(s, 2 * M::NS), lo, n, V);
+        else
+          tape_state<M, G, C>(tape_at(s, 0), fb.n_total, lo, n, V, g);
       }
       if (busy) {
         const double t0 = half_start(row, half), dt = row[2];
@@ -266,11 +295,7 @@ __device__ __forceinline__ void fibre_steps(const DevFibers &fb, const FibreStim
           fibre_heun<M, G, E, C>(V, g, p, t0 + j * dt, dt, on, inset, st, on && !st.clamp ? st.amplitude[f] : 0.0);
         }
       }
-      if (TAPE && tr.tape && !half) {
-#pragma unroll
-        for (int k = 0; k < C; k++)
-          if (lo + k < n) tape_store<M::NS>(tr, fb.n_total, s, M::NS, off + lo + k, V[k], g[k], M::NS);
-      }
+      if (TAPE && tr.tape && !half) tape_state<M, G, C>(tape_at(s, M::NS), fb.n_total, lo, n, V, g);
       if (half && TAPE && sensor) {
 #pragma unroll
         for (int k = 0; k < C; k++)

@@ -19,7 +19,6 @@
 #include <vector>
 
 #include "../../include/opendihu_fms.h"
-#include "fms_adjoint.h"
 #include "fms_fused.h"
 #include "fms_kernels.h"
 #include "fms_parts.h"
@@ -1651,13 +1650,14 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
     const int F = s->F, S = s->n_sensors, K = s->adj_K, Kc = s->adj_interval, n0D = s->adj_n0D;
     const int ie = s->scheme == FMS_IMPLICIT_EULER;
     int rc;
+    // at most 4 nodes per thread; 1024 threads would leave 128 registers each
+    const int T = s->tune_adjoint_threads == 256 && s->nmax <= 1024 ? 256 : 512;
     long long c1 = 0, c2 = 0, c3 = 0, c4 = 0;
-    if ((rc = ensure(&s->d_lam, c1, 4 * N)) || (rc = ensure(&s->d_gacc, c2, 3 * N)) ||
+    if ((rc = ensure(&s->d_lam, c1, 4 * N)) || (rc = ensure(&s->d_gacc, c2, 4LL * F * T)) ||
         (rc = ensure(&s->d_pfbar, c3, F)) || (rc = ensure(&s->d_grad, c4, 3 * (long long)F)))
       return rc;
     HIP_TRY(hipMemsetAsync(s->d_lam, 0, 4 * N * sizeof(double), s->stream));
-    HIP_TRY(hipMemsetAsync(s->d_gacc, 0, 3 * N * sizeof(double), s->stream));
-    HIP_TRY(hipMemsetAsync(s->d_pfbar, 0, F * sizeof(double), s->stream));
+    HIP_TRY(hipMemsetAsync(s->d_gacc, 0, 4LL * F * T * sizeof(double), s->stream));
     // the whole forward's tape (segment seg at seg * tape_len), or two segment
     // buffers: the recompute of segment seg-1 (stream2) runs beside the reverse
     // of segment seg (stream)
@@ -1690,8 +1690,6 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
     // reverse wave, the streamed kernel's (126) do; both give the same bits
     const int saved_resident = s->tune_resident;
     if (s->tune_adjoint != FMS_ADJOINT_SERIAL) s->tune_resident = 0;
-    constexpr int T = 256;
-    const size_t lds = (size_t)(fms::pcr_lds_doubles<1024>() + 3 * s->nmax) * sizeof(double);
     hipStream_t main_stream = s->stream;
     for (int idx = 0, seg = nseg - 1; seg >= 0; seg--, idx++) {
       const int k0 = seg * L, kc = std::min(L, K - k0);
@@ -1720,30 +1718,21 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
           break;
         }
       }
-      const double *dtr = d_dtraces + (size_t)k0 * F * S;
-      const int prio = !whole && s->tune_adjoint == FMS_ADJOINT_OVERLAP_PRIORITY;
-      const int at = s->tune_adjoint_threads;
-#define FMS_ADJ_LAUNCH(TT, NPT_, MMAX_)                                                                           \
-  hipLaunchKernelGGL((fms::k_adj_fused<E, TT, NPT_, MMAX_>), dim3(F), dim3(TT), lds, s->stream, s->fibers(),       \
-                     s->stim(), tape, s->d_steps + 4 * (size_t)k0, kc, n0D, ie, s->d_sensor_slot, dtr, S, s->d_lam, \
-                     s->d_gacc, s->d_pfbar, prio)
-      if (at == 1024 && s->nmax <= 1024)
-        FMS_ADJ_LAUNCH(1024, 1, 4);
-      else if (at == 1024)
-        FMS_ADJ_LAUNCH(1024, 2, 4);
-      else if (at == 512 && s->nmax <= 1024)
-        FMS_ADJ_LAUNCH(512, 2, 4);
-      else if (at == 512)
-        FMS_ADJ_LAUNCH(512, 4, 4);
-#undef FMS_ADJ_LAUNCH
-      else if (s->nmax <= 4 * T)
-        hipLaunchKernelGGL((fms::k_adj_fused<E, T, 4, 8>), dim3(F), dim3(T), lds, s->stream, s->fibers(), s->stim(),
-                           tape, s->d_steps + 4 * (size_t)k0, kc, n0D, ie, s->d_sensor_slot, dtr, S, s->d_lam,
-                           s->d_gacc, s->d_pfbar, prio);
-      else
-        hipLaunchKernelGGL((fms::k_adj_fused<E, T, 8, 8>), dim3(F), dim3(T), lds, s->stream, s->fibers(), s->stim(),
-                           tape, s->d_steps + 4 * (size_t)k0, kc, n0D, ie, s->d_sensor_slot, dtr, S, s->d_lam,
-                           s->d_gacc, s->d_pfbar, prio);
+      fms::AdjArgs args{};
+      args.fb = s->fibers();
+      args.st = fms::AdjStim{s->stim_mode == FMS_STIM_CURRENT, s->stim_param, s->d_onset, s->d_dur, s->d_amp};
+      args.tape = tape;
+      args.steps = s->d_steps + 4 * (size_t)k0;
+      args.kc = kc;
+      args.n0D = n0D;
+      args.ie = ie;
+      args.sensor_slot = s->d_sensor_slot;
+      args.dtrace = d_dtraces + (size_t)k0 * F * S;
+      args.n_sensors = S;
+      args.lam = s->d_lam;
+      args.acc = s->d_gacc;
+      args.raise_priority = !whole && s->tune_adjoint == FMS_ADJOINT_OVERLAP_PRIORITY;
+      fms::adjoint_launch<E>(T, s->nmax, args, s->stream);
       if (hipGetLastError() != hipSuccess) {
         rc = fail(FMS_ERR_HIP, "adjoint kernel launch failed");
         break;
@@ -1758,7 +1747,8 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
     s->spikes = saved_spikes;
     s->tune_resident = saved_resident;
     if (rc) return rc;
-    hipLaunchKernelGGL(fms::k_adj_reduce, dim3(F), dim3(256), 0, s->stream, s->fibers(), s->d_gacc, s->d_grad);
+    hipLaunchKernelGGL(fms::k_adj_reduce, dim3(F), dim3(256), 0, s->stream, F, T, s->d_gacc, ie ? 1.0 : 0.5, s->d_grad,
+                       s->d_pfbar);
     HIP_TRY(hipGetLastError());
     return 0;
   }

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
+#include "fms_adjoint.h"
 #include "fms_fibre.h"
 #include "fms_model.h"
 
@@ -34,5 +35,11 @@ extern template void fibre_launch<float, ExpApproxFma, false>(int, const FibreLa
 extern template void fibre_launch<float, ExpLibmFma, false>(int, const FibreLaunch &);
 extern template void fibre_launch<double, ExpApproxFma, true>(int, const FibreLaunch &);
 extern template void fibre_launch<double, ExpLibmFma, true>(int, const FibreLaunch &);
+
+// the reverse sweep of one segment (Hodgkin-Huxley only), T threads per fibre: 256 or 512
+template <class E> void adjoint_launch(int T, int nmax, const AdjArgs &a, hipStream_t stream);
+
+extern template void adjoint_launch<ExpApproxFma>(int, int, const AdjArgs &, hipStream_t);
+extern template void adjoint_launch<ExpLibmFma>(int, int, const AdjArgs &, hipStream_t);
 
 }  // namespace fms

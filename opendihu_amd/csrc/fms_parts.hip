@@ -21,6 +21,16 @@ template <class G, class E, bool TAPE> void fibre_launch(int T, const FibreLaunc
   else fibre_launch_shape<G, E, 256, 8, TAPE>(l);
 }
 
+template <class E, int T, int CMAX> void adjoint_launch_threads(int nmax, const AdjArgs &a, hipStream_t stream) {
+  const size_t lds = chunk_lds_doubles<T>((nmax + T - 1) / T) * sizeof(double);
+  hipLaunchKernelGGL((k_adj_steps<E, T, CMAX>), dim3(a.fb.n_fibers), dim3(T), lds, stream, a);
+}
+
+template <class E> void adjoint_launch(int T, int nmax, const AdjArgs &a, hipStream_t stream) {
+  if (T == 256) adjoint_launch_threads<E, 256, 4>(nmax, a, stream);
+  else adjoint_launch_threads<E, 512, 4>(nmax, a, stream);
+}
+
 #if FMS_PART == 0
 template void fibre_launch<double, ExpApproxFma, false>(int, const FibreLaunch &);
 #elif FMS_PART == 1
@@ -33,6 +43,10 @@ template void fibre_launch<float, ExpLibmFma, false>(int, const FibreLaunch &);
 template void fibre_launch<double, ExpApproxFma, true>(int, const FibreLaunch &);
 #elif FMS_PART == 5
 template void fibre_launch<double, ExpLibmFma, true>(int, const FibreLaunch &);
+#elif FMS_PART == 6
+template void adjoint_launch<ExpApproxFma>(int, int, const AdjArgs &, hipStream_t);
+#elif FMS_PART == 7
+template void adjoint_launch<ExpLibmFma>(int, int, const AdjArgs &, hipStream_t);
 #endif
 
 }  // namespace fms
