@@ -64,11 +64,12 @@ template <class E> FMS_HD HHExps hh_exps(double V, HHBases *bases = nullptr) {
     e.xn01 = __builtin_fma(bn, 102.4, -102.4);
   } else {
     e.xm = (V + 50.0) * -0.1;
-    const double xn = (V + 65.0) * -0.1;
-    e.xn01 = xn * 0.1;
+    e.xn01 = (V + 65.0) * -0.01;
+    // the three of slope -1/10 are one exponential times constants (512 x 1001 nodes,
+    // 300 steps: 5.2 -> 4.2 ms; Vm's error against exact arithmetic stays 1.2e-13)
     e.em = E::exp(e.xm);
-    e.en = E::exp(xn);
-    e.ebh = E::exp((V + 45.0) * -0.1);
+    e.en = e.em * 0.22313016014842982;    // exp(-1.5)
+    e.ebh = e.em * 1.6487212707001282;    // exp(0.5)
     e.ebm = E::exp(v75 * (-1.0 / 18));
     e.eah = E::exp(v75 * -0.05);
     e.ebn = E::exp(v75 * 0.0125);
