@@ -132,11 +132,6 @@ static __global__ __launch_bounds__(64) void k_fibre_flags(DevStim st, const dou
   }
 }
 
-// nodes whose Heun steps share a basic block
-#ifndef FIBRE_GROUP
-#define FIBRE_GROUP 1
-#endif
-
 // what the fused kernel needs of the stimulation
 struct FibreStim {
   int clamp;        // the stimulus sets Vm to vstim (firing table), else parameter `param` to the amplitude
@@ -154,28 +149,16 @@ __device__ __forceinline__ void fibre_heun(double *V, G (*g)[M::NS - 1], const d
                                            unsigned inset, const FibreStim &st, double amplitude) {
   if constexpr (std::is_same<M, ModelHH>::value) {
     if (!on || st.clamp || st.param == 0) {
-      constexpr_for<0, C, FIBRE_GROUP>([&](auto k_) {
-        constexpr int k = decltype(k_)::value, Q = k + FIBRE_GROUP <= C ? FIBRE_GROUP : C - k;
-        double p0[Q];
-#pragma unroll
-        for (int q = 0; q < Q; q++) p0[q] = p[0];
-        if (on && !st.clamp) {
-#pragma unroll
-          for (int q = 0; q < Q; q++) p0[q] = (inset >> (k + q)) & 1 ? amplitude : p[0];
-        }
-        hh_step_nodes<G, E, false, Q>(V + k, g + k, p, p0, dt,
+      constexpr_for<0, C, 1>([&](auto k_) {
+        constexpr int k = decltype(k_)::value;
+        double p0[1] = {p[0]};
+        if (on && !st.clamp) p0[0] = (inset >> k) & 1 ? amplitude : p[0];
+        hh_step_nodes<G, E, false, 1>(V + k, g + k, p, p0, dt,
                                       [&](double(*ys)[4]) {
-                                        if (on && st.clamp) {
-#pragma unroll
-                                          for (int q = 0; q < Q; q++)
-                                            ys[q][0] = (inset >> (k + q)) & 1 ? st.vstim : ys[q][0];
-                                        }
+                                        if (on && st.clamp) ys[0][0] = (inset >> k) & 1 ? st.vstim : ys[0][0];
                                       },
                                       nullptr);
-        if (on && st.clamp) {
-#pragma unroll
-          for (int q = 0; q < Q; q++) V[k + q] = (inset >> (k + q)) & 1 ? st.vstim : V[k + q];
-        }
+        if (on && st.clamp) V[k] = (inset >> k) & 1 ? st.vstim : V[k];
       });
       return;
     }
@@ -337,9 +320,6 @@ __device__ __forceinline__ void fibre_steps(const DevFibers &fb, const FibreStim
 
 // waves per SIMD the kernel is compiled for
 template <int T, int CMAX> constexpr int fibre_occupancy() {
-#ifdef FIBRE_OCC
-  return FIBRE_OCC;
-#endif
   return T >= 512 && CMAX <= 4 ? 4 : 2;
 }
 

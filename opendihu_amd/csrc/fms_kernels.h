@@ -20,8 +20,11 @@
 //   k_reaction_fibre  the same with one workgroup per fibre (large models)
 //   k_thomas_serial   one wave per fibre, the reference's Thomas recurrence (bit-exact)
 //   k_thomas_part     one workgroup per fibre, partitioned Thomas + PCR in LDS
+//                     (models of more than 8 states; small models: fms_chunk.h)
 //   k_fused           one workgroup per fibre, many split steps; Vm lives in LDS,
-//                     gates in registers (RESIDENT) or streamed from HBM
+//                     gates in registers (RESIDENT) or streamed from HBM: the serial
+//                     solve of small models, and larger models (fms_fused.h). Small
+//                     models with the partitioned solve: k_fibre (fms_fibre.h)
 #pragma once
 
 #include "fms_math.h"
@@ -764,10 +767,8 @@ __device__ __forceinline__ void serial_solve(double *sc, int n, double *u, const
 // lv: n doubles of Vm in LDS (overwritten with the solution)
 // red: pcr_lds_doubles<T>() doubles of LDS scratch (6 per wave)
 // Requires n >= 2 and ceil(n / min(T, n/2)) <= MMAX. Ends with a barrier.
-// GIVEN_RHS: lv holds the right-hand side itself (adjoint solves) instead of the
-// Vm from which the right-hand side B*Vm is assembled.
 // ----------------------------------------------------------------------------
-template <int T, int MMAX, bool GIVEN_RHS = false>
+template <int T, int MMAX>
 __device__ __forceinline__ void lds_thomas_part(double *lv, int n, const double *h, double prefactor, double dt,
                                                 bool ie, double *red, int tid) {
   static_assert(T % 64 == 0 && T >= 64 && T <= 1024, "the solve works on whole waves");
@@ -786,7 +787,6 @@ __device__ __forceinline__ void lds_thomas_part(double *lv, int n, const double 
       if (k < cnt) {
         double a, b, c, d;
         assemble_row(lo + k, n, lv, h, prefactor, dt, ie, a, b, c, d);
-        if (GIVEN_RHS) d = lv[lo + k];
         if (k < 2) {
           const double rb = recip_nr(b);   // the first two rows share one reciprocal
           aa[k] = a * rb;

@@ -170,15 +170,17 @@ class FiberBatch:
                    reaction_threads: int | None = None, adjoint: int | None = None,
                    adjoint_threads: int | None = None, adjoint_tape: int | None = None) -> None:
         """Schedule knobs. Fused kernel: split steps per launch; gates in registers (1),
-        streamed (0) or auto (-1); threads per fibre workgroup (128 or 256). Split
+        streamed (0) or auto (-1; small models with the partitioned solve always keep
+        them in registers); threads per fibre workgroup (128 or 256; that solve takes
+        512 for fibres of more than 2048 nodes). Split
         kernels: steps per captured hipGraph (0 launches eagerly); for large models
         the reaction with one workgroup per fibre (1) or one lane per node (0); the
         two reaction halves between two solves in one launch (1, default) or one
         launch per half (0); threads per fibre of the per-fibre reaction (256 or 64).
         Adjoint backward: segment recompute beside the reverse sweep (0), the same
         with the reverse sweep's priority raised (1) or the recompute's (3), or one
-        after the other (2); threads per fibre workgroup of the reverse sweep (256,
-        512 or 1024); the adjoint forward records the whole tape (1) or keeps
+        after the other (2); threads per fibre workgroup of the reverse sweep (256 for
+        fibres of up to 1024 nodes, else 512; 1024 runs as 512); the adjoint forward records the whole tape (1) or keeps
         checkpoints that the backward recomputes from (0), or the whole tape when it
         fits in half of the free device memory (-1, default)."""
         for key, value in ((L.FMS_TUNE_STEPS_PER_LAUNCH, steps_per_launch), (L.FMS_TUNE_RESIDENT_GATES, resident_gates),
