@@ -146,14 +146,14 @@ struct FmsSolver {
   // schedule knobs (fms_set_tuning): steps per fused launch, gate residency,
   // threads per fibre workgroup, split steps per captured graph (0: no graph)
   int tune_chunk = 512;
-  int tune_resident = -1;   // -1 auto, 0 stream gates from HBM, 1 keep gates in registers
+  int tune_resident = -1;   // k_fused: -1 auto, 0 stream gates from HBM, 1 keep gates in registers
   int tune_threads = 256;
   int tune_graph = 0;
   int tune_reaction_fibre = 1;   // split kernels, large models: one workgroup per fibre for the reaction
   int tune_pair = 1;   // split kernels: the two reaction halves between two solves in one launch
   int tune_reaction_threads = 256;   // split kernels, per-fibre reaction: threads per fibre workgroup (64 or 256)
   int tune_adjoint = FMS_ADJOINT_SERIAL;    // adjoint backward: recompute beside the reverse sweep or before it
-  int tune_adjoint_threads = 512;           // threads per fibre workgroup of the reverse sweep (256, 512, 1024)
+  int tune_adjoint_threads = 512;           // reverse sweep: 256 threads per fibre (up to 1024 nodes), else 512
   int tune_adjoint_tape = FMS_ADJOINT_TAPE_AUTO;   // the forward records the whole tape, or checkpoints
 
   // per-kernel timing (fms_set_tuning(FMS_TUNE_PROFILE_KERNELS)): a start and
@@ -1685,9 +1685,10 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
     }
     const int saved_spikes = s->spikes;
     s->spikes = 0;
-    // a recompute beside the reverse sweep streams its gates: the resident-gate
-    // kernel's registers (194 per lane for HH) do not fit on a SIMD beside a
-    // reverse wave, the streamed kernel's (126) do; both give the same bits
+    // the serial solve's recompute beside the reverse sweep streams its gates: the
+    // resident-gate kernel's registers (194 per lane for HH) do not fit on a SIMD
+    // beside a reverse wave, the streamed kernel's (126) do; both give the same
+    // bits. The partitioned solve's kernel keeps its gates and ignores the switch.
     const int saved_resident = s->tune_resident;
     if (s->tune_adjoint != FMS_ADJOINT_SERIAL) s->tune_resident = 0;
     hipStream_t main_stream = s->stream;
@@ -1707,7 +1708,11 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
         tr.tape = tape;
         tr.raise_priority = s->tune_adjoint == FMS_ADJOINT_OVERLAP_RECOMPUTE_PRIORITY;
         const long long save = s->step_counter;
-        if (!rc) rc = launch_fused<double, E>(s, s->d_steps + 4 * (size_t)k0, kc, n0D, tr);
+        // the forward's kernels, so that the recomputed tape has the forward's bits
+        if (!rc)
+          rc = with_exp(s, [&](auto e) {
+            return launch_fused<double, decltype(e)>(s, s->d_steps + 4 * (size_t)k0, kc, n0D, tr);
+          });
         s->step_counter = save;
         if (!rc && hipEventRecord(s->adj_ev[2 + buf], s->stream) != hipSuccess) rc = FMS_ERR_HIP;
         s->stream = main_stream;

@@ -230,3 +230,23 @@ def test_gradient_nodes_per_thread(scheme, lengths, threads):
     is within 1e-13 of itself in 80-bit arithmetic here"""
     for f, g, ref in _gradients(lengths, scheme, threads, lambda k: k // 2 + np.array([-2, 0, 3]), 12):
         np.testing.assert_allclose(g, ref, rtol=1e-9, err_msg=f"fibre {f}")
+
+
+@pytest.mark.parametrize("thomas", ["serial", "partitioned"])
+def test_recomputed_segments_have_the_forward_bits(thomas):
+    """whole tape and checkpoints: the same gradient for either solve"""
+    from opendihu_amd.adjoint import AdjointProblem
+    from opendihu_amd.fibers import FiberBatch
+    mesh = _mesh([30, 300, 700])
+    stim = _pulse(mesh["n_nodes"])
+    theta = np.stack([np.full(3, 120.0), np.full(3, 36.0), np.full(3, 0.3), mesh["prefactor"] * AM * CM], 1)
+    sensors = (mesh["n_nodes"][:, None] // 2 + np.array([[-2, 3]])).astype(np.int32)
+    grads = []
+    for tape in ("whole", "segments"):
+        b = FiberBatch(**mesh, scheme="CN", kernels="fused", thomas=thomas)
+        b.set_current_stimulation(**stim)
+        prob = AdjointProblem(b, _rows(70), sensors, checkpoint_interval=16, tape=tape)
+        tr = prob.forward(theta)
+        grads.append(prob.backward(np.random.default_rng(6).standard_normal(tr.shape)))
+    assert np.isfinite(grads[0]).all() and (grads[0] != 0).all()
+    np.testing.assert_array_equal(grads[0], grads[1])
