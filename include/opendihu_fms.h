@@ -182,7 +182,8 @@ int fms_last_error(char *buf, int len);
 
 /* schedule knobs of the fused kernel (the autotuner's search space) */
 #define FMS_TUNE_STEPS_PER_LAUNCH 1   /* split steps per fused launch (default 512) */
-#define FMS_TUNE_RESIDENT_GATES 2     /* -1 auto, 0 stream gates from HBM, 1 keep them in registers */
+#define FMS_TUNE_RESIDENT_GATES 2     /* -1 auto, 0 stream gates from HBM, 1 keep them in registers;
+                                         small models with the partitioned solve always keep them */
 /* onlyComputeIfHasBeenStimulated (0/1, default 0): a fibre's reaction runs from
    the Heun step of its first stimulation on; diffusion always runs */
 #define FMS_TUNE_ONLY_IF_STIMULATED 3
@@ -215,16 +216,16 @@ int fms_set_point_buffer_order(FmsSolver *solver, int width, const int *nmj /* [
    of the next segment runs on a second stream beside the reverse of this one;
    _OVERLAP_PRIORITY: the same, the reverse sweep's waves with raised issue
    priority; _SERIAL (default): recompute and reverse one after the other on the
-   solver's stream. A recompute beside the reverse sweep streams its gates from
-   HBM (fewer registers, so that it shares the SIMDs with the sweep); a serial
-   one uses the solver's fused schedule. Same arithmetic, same gradients. */
+   solver's stream. With the serial solve, a recompute beside the reverse sweep
+   streams its gates from HBM (fewer registers, so that it shares the SIMDs with
+   the sweep). Same arithmetic, same gradients. */
 #define FMS_TUNE_ADJOINT 10
 #define FMS_ADJOINT_OVERLAP 0
 #define FMS_ADJOINT_OVERLAP_PRIORITY 1
 #define FMS_ADJOINT_SERIAL 2
 #define FMS_ADJOINT_OVERLAP_RECOMPUTE_PRIORITY 3   /* beside it, the recompute's waves with raised priority */
-/* threads per fibre workgroup of the adjoint's reverse sweep: 256, 512
-   (default) or 1024 (fewer nodes per thread, more waves per SIMD). The prefactor
+/* threads per fibre workgroup of the adjoint's reverse sweep: 512
+   (default; 1024 runs as 512) or 256 (taken for fibres of up to 1024 nodes). The prefactor
    gradient is summed per wave and then over the waves, so its last bits depend
    on this number. */
 #define FMS_TUNE_ADJOINT_THREADS 11
@@ -265,8 +266,9 @@ int fms_graph_counts(FmsSolver *solver, long long *captures, long long *replays)
 
 /* Autotuner (no counterpart in the reference, which has one fixed CPU schedule
    and an OpenMP-offload loop): times every schedule that gives bit-identical
-   states on this batch - fused kernel with gates resident or streamed, 128 or
-   256 threads per fibre, 64 or 512 steps per launch; with allow_split also the
+   states on this batch - fused kernel with 64, 256 or 512 steps per launch (serial
+   solve: gates resident or streamed, 128 or 256 threads per fibre, 64 or 512
+   steps); with allow_split also the
    split kernels launched eagerly or replayed as hipGraphs of 8 or 32 steps
    (models of > 8 states: reaction per fibre with 256 or 64 threads, or per node,
    eager or graphs of 8) -

@@ -2101,13 +2101,16 @@ std::vector<Schedule> candidates(const FmsSolver *s, int allow_split) {
   const bool fused_ok = !(s->nmax > 2048 && s->thomas == FMS_THOMAS_SERIAL) && s->nmax <= 4096;
   const int pf = s->tune_reaction_fibre, rt = s->tune_reaction_threads;
   if (fused_ok) {
-    if (small) {
+    if (small && s->thomas == FMS_THOMAS_PARTITIONED) {
+      // the gates stay in registers: only the launches' length is left
+      for (int chunk : {64, 256, 512}) v.push_back({FMS_KERNELS_FUSED, chunk, 1, 256, 0, pf, rt});
+    } else if (small) {
       for (int chunk : {64, 512}) {
         v.push_back({FMS_KERNELS_FUSED, chunk, 1, 256, 0, pf, rt});
         v.push_back({FMS_KERNELS_FUSED, chunk, 0, 256, 0, pf, rt});
         // the partitioned solve's elimination order depends on the threads per
         // fibre, so 128-thread schedules are bit-identical only with the serial solve
-        if (s->thomas == FMS_THOMAS_SERIAL && s->nmax <= 1024) {
+        if (s->nmax <= 1024) {
           v.push_back({FMS_KERNELS_FUSED, chunk, 1, 128, 0, pf, rt});
           v.push_back({FMS_KERNELS_FUSED, chunk, 0, 128, 0, pf, rt});
         }
