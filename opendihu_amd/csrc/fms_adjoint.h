@@ -113,12 +113,13 @@ __device__ __forceinline__ HHLin hh_linearize(const double *y, const double *p) 
   const HHExps e = hh_exps<E>(V, &b);
   double im, in, ih;
   hh_inverses(e, im, in, ih);
-  const double am = e.xm * im, an = e.xn01 * in;
+  const HHQuotients qu = hh_quotients<E>(e, im, in, ih);
+  const double am = qu.am, an = qu.an, bh = qu.bh;
   const double ah = 0.07 * e.eah, bm = 4.0 * e.ebm, bn = 0.125 * e.ebn;
-  const double sm = __builtin_fma(4.0, e.ebm, am), sh = ah + ih, sn = __builtin_fma(0.125, e.ebn, an);
-  L.r[1] = __builtin_fma(-sm, m, am);
-  L.r[2] = __builtin_fma(-sh, h, ah);
-  L.r[3] = __builtin_fma(-sn, n, an);
+  const double sm = __builtin_fma(4.0, e.ebm, am), sh = ah + bh, sn = __builtin_fma(0.125, e.ebn, an);
+  L.r[1] = hh_gate_rate<E>(am, 4.0, e.ebm, sm, m);
+  L.r[2] = hh_gate_rate<E>(ah, 1.0, bh, sh, h);
+  L.r[3] = hh_gate_rate<E>(an, 0.125, e.ebn, sn, n);
   const double m2 = m * m, m3 = m2 * m, m3h = m3 * h, n2 = n * n, n4 = n2 * n2;
   const double gm3h = p[1] * m3h, gn4 = p[2] * n4;
   const double vna = V - 40.0, vk = V + 87.0, vl = V + (75.0 - 10.6130);
@@ -138,7 +139,7 @@ __device__ __forceinline__ HHLin hh_linearize(const double *y, const double *p) 
   const double dun = near_n ? dus : in * __builtin_fma(-10.0 * an, e.en * ib.n, 1.0);
   const double dam = -0.1 * dum, dan = -0.01 * dun;
   const double dbm = bm * ib.bm * (-1.0 / 18.0), dah = ah * ib.ah * (-1.0 / 20.0);
-  const double dbh = ih * ih * (e.ebh * ib.bh) * 0.1, dbn = bn * ib.bn * (1.0 / 80.0);
+  const double dbh = bh * bh * (e.ebh * ib.bh) * 0.1, dbn = bn * ib.bn * (1.0 / 80.0);
   L.f0V = -(gm3h + gn4 + p[3]);
   const double gv = -p[1] * vna;
   L.f0m = 3.0 * m2 * h * gv;

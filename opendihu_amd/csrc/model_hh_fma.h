@@ -9,15 +9,23 @@
 //    which the ten squarings multiply by 1024, stays the only one.
 //  * alpha_m = x/(E(x) - 1) takes x = 1024 (base - 1), one exact instruction, and
 //    alpha_n likewise.
-//  * The three quotients share one reciprocal.
-//  * d gate/dt = alpha - (alpha + beta) gate, currents and Heun updates as fused
-//    multiply-adds.
+//  * The three quotients share one reciprocal; under the device's exp, whose error is
+//    as small as a product's, each is corrected by its remainder.
+//  * d gate/dt = alpha - (alpha + beta) gate (under the device's exp
+//    alpha (1 - gate) - beta gate), currents and Heun updates as fused multiply-adds.
 //
 // About 110 FP64 instructions per right-hand side instead of 175; FP64 issue is what
-// bounds the kernels. 4096 fibres of 400-2000 nodes, 1000 steps and the states read
-// back: 183 -> 156 ms (mixed 113 -> 95 ms); 512 x 1001 with the device's exp, 300
-// steps: 8.0 -> 7.3 ms. The error against exact arithmetic falls (Vm of the same
-// 4096 fibres, relative L2: 5e-12 -> 2e-13).
+// bounds the kernels. In kernels that are otherwise the same, 4096 fibres of 400-2000
+// nodes, 1000 steps and the states read back: 183 -> 156 ms (mixed 113 -> 95 ms).
+// Mean errors of the rates against 80-bit arithmetic, Vm from -90 to 40 mV, as a share
+// of the model form's, on the device: dV/dt 0.89, dm/dt, dh/dt and dn/dt 0.84, 1.00 and
+// 0.80 (approximate exponential), 0.95, 1.00 and 0.96 (device's exp; no larger in any of
+// the bands -90..-70, -70..-60, -55..-45 and -40..40 mV). With the approximate
+// exponential alpha_m's x has the base's error of 1e-13: what it cancels around -50 mV
+// is most of the former error, at -40..40 mV it is 4 times the former 3e-15 relative.
+// Under the device's exp, en and ebh as multiples of em were 24 % faster (512 x 1001
+// nodes, 300 steps: 4.3 against 5.4 ms; model form and its kernels 8.0) but gave dn/dt
+// 1.75 times the model form's mean error and 9.5 times its rms one, around -65 mV.
 #pragma once
 
 #include "fms_math.h"
@@ -43,6 +51,9 @@ struct HHBases {
   double m, n, bh, bm, ah, bn;
 };
 
+// v (c + c_lo)
+FMS_HD double hh_two_term(double v, double c, double c_lo) { return __builtin_fma(v, c, v * c_lo); }
+
 template <class E> FMS_HD HHExps hh_exps(double V, HHBases *bases = nullptr) {
   HHExps e;
   const double v75 = V + 75.0;
@@ -63,16 +74,17 @@ template <class E> FMS_HD HHExps hh_exps(double V, HHBases *bases = nullptr) {
     e.xm = __builtin_fma(bm, 1024.0, -1024.0);
     e.xn01 = __builtin_fma(bn, 102.4, -102.4);
   } else {
-    e.xm = (V + 50.0) * -0.1;
-    e.xn01 = (V + 65.0) * -0.01;
-    // the three of slope -1/10 are one exponential times constants (512 x 1001 nodes,
-    // 300 steps: 5.2 -> 4.2 ms; Vm's error against exact arithmetic stays 1.2e-13)
-    e.em = E::exp(e.xm);
-    e.en = e.em * 0.22313016014842982;    // exp(-1.5)
-    e.ebh = e.em * 1.6487212707001282;    // exp(0.5)
-    e.ebm = E::exp(v75 * (-1.0 / 18));
-    e.eah = E::exp(v75 * -0.05);
+    // six exponentials, each of its own argument: the quotient by the slope as the
+    // product with its reciprocal in two terms, which is correctly rounded but for ties
+    const double v50 = V + 50.0, v65 = V + 65.0, v45 = V + 45.0;
+    e.em = E::exp(hh_two_term(v50, -0.1, 5.551115123125783e-18));
+    e.en = E::exp(hh_two_term(v65, -0.1, 5.551115123125783e-18));
+    e.ebh = E::exp(hh_two_term(v45, -0.1, 5.551115123125783e-18));
+    e.ebm = E::exp(hh_two_term(v75, -1.0 / 18, -3.0839528461809902e-18));
+    e.eah = E::exp(hh_two_term(v75, -0.05, 2.7755575615628915e-18));
     e.ebn = E::exp(v75 * 0.0125);
+    e.xm = v50 * -0.1;
+    e.xn01 = v65 * -0.01;
   }
   return e;
 }
@@ -106,17 +118,42 @@ FMS_HD void hh_inverses(const HHExps &e, double &im, double &in, double &ih) {
   in = rh * dm;
 }
 
+// the device's exponential leaves the quotients and the sums of a rate as the largest
+// errors of the rates; the approximate one's 1024-fold base error is above them
+template <class E> constexpr bool hh_exact() { return !std::is_base_of<ExpApprox, E>::value; }
+
+// alpha_m, alpha_n and beta_h from the shared reciprocal's im, in, ih
+struct HHQuotients {
+  double am, an, bh;
+};
+template <class E> FMS_HD HHQuotients hh_quotients(const HHExps &e, double im, double in, double ih) {
+  HHQuotients q{e.xm * im, e.xn01 * in, ih};
+  if constexpr (hh_exact<E>()) {
+    // one step on the remainder each: the errors of the shared reciprocal's products go
+    q.am = __builtin_fma(__builtin_fma(-(e.em - 1.0), q.am, e.xm), im, q.am);
+    q.an = __builtin_fma(__builtin_fma(-(e.en - 1.0), q.an, e.xn01), in, q.an);
+    q.bh = __builtin_fma(__builtin_fma(-(e.ebh + 1.0), ih, 1.0), ih, ih);
+  }
+  return q;
+}
+
+// alpha (1 - x) - beta x with beta = cb eb (cb a power of two), s = alpha + beta
+template <class E> FMS_HD double hh_gate_rate(double alpha, double cb, double eb, double s, double x) {
+  if constexpr (hh_exact<E>()) return __builtin_fma(alpha, 1.0 - x, -((cb * eb) * x));
+  return __builtin_fma(-s, x, alpha);
+}
+
 // rates r[4] at (V, m, h, n), dV/dt without the stimulus; ALG: the algebraics of the model file in a[9]
 template <class E, bool ALG>
 FMS_HD void hh_rates_fused(double V, double m, double h, double n, const double *p, double *r, double *a) {
   const HHExps e = hh_exps<E>(V);
   double im, in, ih;
   hh_inverses(e, im, in, ih);
-  const double am = e.xm * im, an = e.xn01 * in;
-  const double ah = 0.07 * e.eah;
-  r[1] = __builtin_fma(-__builtin_fma(4.0, e.ebm, am), m, am);
-  r[2] = __builtin_fma(-(ah + ih), h, ah);
-  r[3] = __builtin_fma(-__builtin_fma(0.125, e.ebn, an), n, an);
+  const HHQuotients q = hh_quotients<E>(e, im, in, ih);
+  const double am = q.am, an = q.an, ah = 0.07 * e.eah;
+  r[1] = hh_gate_rate<E>(am, 4.0, e.ebm, __builtin_fma(4.0, e.ebm, am), m);
+  r[2] = hh_gate_rate<E>(ah, 1.0, q.bh, ah + q.bh, h);
+  r[3] = hh_gate_rate<E>(an, 0.125, e.ebn, __builtin_fma(0.125, e.ebn, an), n);
   const double gm3h = p[1] * (m * m * m * h), n2 = n * n, gn4 = p[2] * (n2 * n2);
   const double vna = V - 40.0, vk = V + 87.0, vl = V + (75.0 - 10.6130);
   r[0] = __builtin_fma(-gm3h, vna, __builtin_fma(-gn4, vk, -(p[3] * vl)));
@@ -127,7 +164,7 @@ FMS_HD void hh_rates_fused(double V, double m, double h, double n, const double 
     a[3] = an;
     a[4] = gn4 * vk;
     a[5] = 4.0 * e.ebm;
-    a[6] = ih;
+    a[6] = q.bh;
     a[7] = 0.125 * e.ebn;
     a[8] = p[3] * vl;
   }
