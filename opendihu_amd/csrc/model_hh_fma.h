@@ -22,7 +22,7 @@
 // 0.80 (approximate exponential), 0.95, 1.00 and 0.96 (device's exp; no larger in any of
 // the bands -90..-70, -70..-60, -55..-45 and -40..40 mV). With the approximate
 // exponential alpha_m's x has the base's error of 1e-13: what it cancels around -50 mV
-// is most of the former error, at -40..40 mV it is 4 times the former 3e-15 relative.
+// is most of the former error; at -40..40 mV dm/dt has 4 times its small former one.
 // Under the device's exp, en and ebh as multiples of em were 24 % faster (512 x 1001
 // nodes, 300 steps: 4.3 against 5.4 ms; model form and its kernels 8.0) but gave dn/dt
 // 1.75 times the model form's mean error and 9.5 times its rms one, around -65 mV.
@@ -107,12 +107,21 @@ FMS_HD HHBases hh_inverse_bases(const HHBases &b) {
   return r;
 }
 
-// 1/(em - 1), 1/(en - 1) and 1/(ebh + 1) from one reciprocal
+// 1/(em - 1), 1/(en - 1) and 1/(ebh + 1) from one reciprocal, for every Vm at which the
+// three are finite: where their product overflows (below -2400 mV; above 23000 mV with
+// the approximate exponential) each of the three is above 1e102 in size, the
+// reciprocal is 0, not the Newton steps' NaN, and so are the quotients, multiplied by
+// one factor at a time. (The two instructions cost 0 to 3 %: 4096 x 1000 nodes 66 -> 67
+// us per step, 256 x 1000 6.9 -> 7.0, 1 x 100 2.75 -> 2.70. A branch to three
+// reciprocals spilled 611 registers instead of 43, one per Heun step cost 5 %.)
 FMS_HD void hh_inverses(const HHExps &e, double &im, double &in, double &ih) {
   const double dm = e.em - 1.0, dn = e.en - 1.0, dh = e.ebh + 1.0;
-  const double dmn = dm * dn;
-  const double r = recip_nr(dmn * dh);
-  ih = r * dmn;
+  const double p = (dm * dn) * dh;
+  double r = recip_nr(p);
+#if defined(__HIP_DEVICE_COMPILE__)
+  r = __builtin_amdgcn_div_fixup(r, p, 1.0);
+#endif
+  ih = (r * dm) * dn;
   const double rh = r * dh;
   im = rh * dn;
   in = rh * dm;

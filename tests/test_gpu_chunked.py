@@ -250,3 +250,32 @@ def test_recomputed_segments_have_the_forward_bits(thomas):
         grads.append(prob.backward(np.random.default_rng(6).standard_normal(tr.shape)))
     assert np.isfinite(grads[0]).all() and (grads[0] != 0).all()
     np.testing.assert_array_equal(grads[0], grads[1])
+
+
+@pytest.mark.parametrize("exp,vm", [("libm", -2500.0), ("libm", -6900.0), ("approx", -2800.0), ("approx", -10100.0),
+                                    ("approx", 24000.0)])
+def test_far_from_rest(exp, vm):
+    """where the product of the reaction's denominators overflows, its rates stay finite:
+    Heun steps so short that the states keep the serial run's values (1e-12), the
+    gradient's sums finite"""
+    from opendihu_amd.adjoint import AdjointProblem
+    from opendihu_amd.fibers import FiberBatch
+    mesh = _mesh([2, 70])
+    rows = _rows(4)
+    rows[:, 2] = 1e-200
+    runs = []
+    for kernels, thomas in (("fused", "serial"), ("fused", "partitioned"), ("split", "partitioned")):
+        b = FiberBatch(**mesh, scheme="CN", kernels=kernels, thomas=thomas, exp_mode=exp)
+        b.set_state(0, np.full(72, vm))
+        b.advance_schedule(rows)
+        runs.append(b.get_states())
+    assert np.isfinite(runs[0]).all()
+    for r in runs[1:]:
+        np.testing.assert_allclose(r, runs[0], rtol=1e-12)
+    b = FiberBatch(**mesh, scheme="CN", kernels="fused", thomas="partitioned", exp_mode=exp)
+    b.set_state(0, np.full(72, vm))
+    b.set_current_stimulation(**_pulse(mesh["n_nodes"]))
+    theta = np.stack([np.full(2, 120.0), np.full(2, 36.0), np.full(2, 0.3), mesh["prefactor"] * AM * CM], 1)
+    prob = AdjointProblem(b, rows, np.array([[0, 1], [5, 69]], np.int32))
+    tr = prob.forward(theta)
+    assert np.isfinite(tr).all() and np.isfinite(prob.backward(np.ones_like(tr))).all()

@@ -245,6 +245,13 @@ template <class E, class EF> static void errors(double lo, double hi, int count,
     }
   }
 }
+// rates at gates 1/2: the model form's in out[0..3], the fused form's in out[4..7]
+extern "C" void rates_at(double V, int approx, double *out) {
+  const double y[4] = {V, 0.5, 0.5, 0.5}, p[4] = {0, 120, 36, 0.3};
+  approx ? model_form<ExpApprox>(y, p, out) : model_form<ExpLibm>(y, p, out);
+  approx ? hh_rates_fused<ExpApproxFma, false>(y[0], y[1], y[2], y[3], p, out + 4, nullptr)
+         : hh_rates_fused<ExpLibmFma, false>(y[0], y[1], y[2], y[3], p, out + 4, nullptr);
+}
 extern "C" void rate_errors(double lo, double hi, int approx, int count, double *out) {
   approx ? errors<ExpApprox, ExpApproxFma>(lo, hi, count, out) : errors<ExpLibm, ExpLibmFma>(lo, hi, count, out);
 }
@@ -272,6 +279,18 @@ def test_fused_reaction_is_as_accurate_as_the_model_form(fused_model, exp, lo, h
     fused_model.rate_errors(ctypes.c_double(lo), ctypes.c_double(hi), int(exp == "approximate"), 200000, P(out, _dp))
     assert (out[:4] > 0).all()
     assert (out[4:] <= 1.02 * out[:4]).all(), out[4:] / out[:4]
+
+
+@pytest.mark.parametrize("exp,vm", [("libm", -2500.0), ("libm", -6900.0), ("libm", 20000.0), ("approximate", -2800.0),
+                                    ("approximate", -10100.0), ("approximate", 24000.0), ("approximate", 30000.0)])
+def test_fused_reaction_far_from_rest(fused_model, exp, vm):
+    """finite rates wherever the model form's are: the product of the quotients'
+    denominators overflows here. 1e-10: an exponential's base error to the 1024th power,
+    a few 1e-13; 1e-98: x of at most 3e3 times a quotient below 1e-102, which is 0 here"""
+    out = np.zeros(8)
+    fused_model.rates_at(ctypes.c_double(vm), int(exp == "approximate"), P(out, _dp))
+    assert np.isfinite(out[:4]).all()
+    np.testing.assert_allclose(out[4:], out[:4], rtol=1e-10, atol=1e-98)
 
 
 @pytest.mark.parametrize("model", ["hh", SHORTEN, "tk2014"])
