@@ -189,6 +189,7 @@ struct AdjStim {
   int on;       // pulses are set
   int param;    // the stimulus parameter
   const double *onset, *duration, *amplitude;   // [F]
+  const int *vc_centre;   // point-buffer order: [F], negative on fibres that are never stimulated; else null
 };
 
 // reverse of one reaction half of a node from its state y0 at t0: l in: adjoint of
@@ -256,7 +257,8 @@ __device__ __forceinline__ void adj_steps(const AdjArgs &a, int f, int off, int 
   int slot[C];
   unsigned inset = 0;
   {
-    const int sb = a.fb.stim_begin[f], se = a.fb.stim_end[f];
+    const bool checked = !a.st.vc_centre || a.st.vc_centre[f] >= 0;
+    const int sb = a.fb.stim_begin[f], se = checked ? a.fb.stim_end[f] : sb;
 #pragma unroll
     for (int q = 0; q < C; q++) {
       // threads past the fibre's end shadow its last node with a zero adjoint

@@ -48,8 +48,8 @@ static __global__ __launch_bounds__(64) void k_fibre_flags(DevStim st, const dou
   const bool only = st.only_if_stimulated != 0;
   bool hb = st.has_been[f] != 0;
   const bool hb_start = hb;
-  const bool table = st.mode == 1;
-  double freq = 0, repeat = 0, begin = 0, last = 0, jit = 0, onset = 0, duration = 0;
+  const bool checked = stim_checked(st, f), table = checked && st.mode == 1;
+  double freq = 0, repeat = 0, begin = 0, last = 0, jit = 0;
   int col = 0, jidx = 0, currently = 0;
   if (table) {
     freq = st.freq[f];
@@ -96,7 +96,7 @@ static __global__ __launch_bounds__(64) void k_fibre_flags(DevStim st, const dou
         }
         done = first + 1;
       }
-    } else if (st.mode == 2) {
+    } else if (checked && st.mode == 2) {
       stim = active && current_on(st, f, t);
     }
     const unsigned long long m = __builtin_amdgcn_ballot_w64(stim != 0);

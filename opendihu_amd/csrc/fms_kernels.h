@@ -172,6 +172,9 @@ __device__ __forceinline__ int current_on(const DevStim &s, int f, double t) {
   return t >= s.onset[f] - 1e-13 && t < s.onset[f] + s.duration[f] - 1e-13;
 }
 
+// a fibre without a centre buffer: the reference never checks its stimulation
+__device__ __forceinline__ bool stim_checked(const DevStim &s, int f) { return s.vc_width <= 0 || s.vc_centre[f] >= 0; }
+
 // per Heun step flag byte: bit 0 = stimulate, bit 1 = compute the reaction
 // (the fibre has been stimulated by this step), bit 2 = the fibre had been
 // stimulated before the reaction half began (point-buffer order)
@@ -179,8 +182,8 @@ constexpr unsigned char FLAG_STIM = 1, FLAG_COMPUTE = 2, FLAG_HB0 = 4;
 
 __device__ __forceinline__ unsigned char stim_flag(const DevStim &s, int f, double t) {
   int stim = 0;
-  if (s.vc_width > 0 && s.vc_centre[f] < 0) {
-    // no centre buffer: the reference never checks this fibre's stimulation
+  if (!stim_checked(s, f)) {
+    // neither stimulated nor its state machine advanced
   } else if (s.mode == 1) {
     stim = stim_check(s, f, t);
   } else if (s.mode == 2) {

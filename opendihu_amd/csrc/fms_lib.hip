@@ -1725,7 +1725,8 @@ template <class E> int adjoint_backward_core(FmsSolver *s, const double *d_dtrac
       }
       fms::AdjArgs args{};
       args.fb = s->fibers();
-      args.st = fms::AdjStim{s->stim_mode == FMS_STIM_CURRENT, s->stim_param, s->d_onset, s->d_dur, s->d_amp};
+      args.st = fms::AdjStim{s->stim_mode == FMS_STIM_CURRENT, s->stim_param, s->d_onset, s->d_dur, s->d_amp,
+                             s->vc_width > 0 ? s->d_vc_centre : nullptr};
       args.tape = tape;
       args.steps = s->d_steps + 4 * (size_t)k0;
       args.kc = kc;
