@@ -188,8 +188,8 @@ int fms_last_error(char *buf, int len);
    the Heun step of its first stimulation on; diffusion always runs */
 #define FMS_TUNE_ONLY_IF_STIMULATED 3
 #define FMS_TUNE_THREADS 4            /* threads per fibre workgroup of the fused kernel: 256 (default) or 128;
-                                         small models with the partitioned solve take 128 up to 1024 nodes
-                                         and 512 above 2048 */
+                                         small models with the partitioned solve, in the split kernels too,
+                                         take 128 up to 1024 nodes and 512 above 2048 */
 #define FMS_TUNE_GRAPH_STEPS 5        /* split kernels: steps per captured hipGraph, 0 = launch eagerly (default) */
 #define FMS_TUNE_REACTION_PER_FIBRE 6 /* split kernels, models of > 8 states: reaction with one workgroup per
                                          fibre (1, default) or one lane per node over the whole batch (0) */

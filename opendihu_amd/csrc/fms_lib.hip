@@ -541,7 +541,8 @@ std::vector<unsigned char> graph_signature(const FmsSolver *s, int gsteps, int n
   struct {
     const void *vm, *gates, *flags, *cursor, *cA, *dA, *vprev, *sfirst, *scount;
     double vstim, spike_th;
-    int spikes, n0D, gsteps, thomas, scheme, nmax, g_is_double, e_is_approx, pair, per_fibre, rthreads;
+    int spikes, n0D, gsteps, thomas, scheme, nmax, g_is_double, e_is_approx, pair, per_fibre, rthreads,
+        cthreads;
   } k;
   memset(&k, 0, sizeof(k));
   k.vm = s->d_vm; k.gates = s->d_gates; k.flags = s->d_flags; k.cursor = s->d_cursor;
@@ -549,6 +550,7 @@ std::vector<unsigned char> graph_signature(const FmsSolver *s, int gsteps, int n
   k.vstim = s->vstim; k.spike_th = s->spike_th; k.spikes = s->spikes; k.n0D = n0D; k.gsteps = gsteps;
   k.thomas = s->thomas; k.scheme = s->scheme; k.nmax = s->nmax;
   k.pair = s->tune_pair; k.per_fibre = s->tune_reaction_fibre; k.rthreads = s->tune_reaction_threads;
+  k.cthreads = chunked_model() && s->thomas == FMS_THOMAS_PARTITIONED ? chunk_threads(s) : 0;
   k.g_is_double = std::is_same<G, double>::value;
   k.e_is_approx = std::is_base_of<fms::ExpApprox, E>::value;
   std::vector<unsigned char> sig(sizeof(fb) + sizeof(st) + sizeof(k));

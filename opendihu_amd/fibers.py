@@ -171,8 +171,9 @@ class FiberBatch:
                    adjoint_threads: int | None = None, adjoint_tape: int | None = None) -> None:
         """Schedule knobs. Fused kernel: split steps per launch; gates in registers (1),
         streamed (0) or auto (-1; small models with the partitioned solve always keep
-        them in registers); threads per fibre workgroup (128 or 256; that solve takes
-        128 for fibres of up to 1024 nodes only and 512 above 2048). Split
+        them in registers); threads per fibre workgroup (128 or 256; that solve, in the
+        split kernels too, takes 128 for fibres of up to 1024 nodes only and 512 above
+        2048). Split
         kernels: steps per captured hipGraph (0 launches eagerly); for large models
         the reaction with one workgroup per fibre (1) or one lane per node (0); the
         two reaction halves between two solves in one launch (1, default) or one

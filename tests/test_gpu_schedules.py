@@ -119,6 +119,23 @@ def test_graph_follows_stimulation_and_spike_changes():
     assert out[1][2]["captures"] == 1 and out[1][3]["captures"] == 2
 
 
+def test_graph_recaptures_when_the_threads_change():
+    """the partitioned solve's partition follows the threads per fibre: a graph captured
+    with others is not replayed, and the steps equal the eager launches' bit for bit"""
+    mesh, stim = uneven(6, lo=300, hi=900, seed=3)
+    out = []
+    for gs in (0, 8):
+        g = _batch(mesh, scheme="CN", kernels="split", thomas="partitioned")
+        g.set_tuning(graph_steps=gs)
+        g.set_current_stimulation(**stim)
+        for k, threads in enumerate((256, 128, 128, 256)):
+            g.set_tuning(threads=threads)
+            g.advance(k * 0.1, 1e-3, 100)
+        out.append((g.get_states(), g.graph_counts()))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[1][1]["captures"] == 3
+
+
 @pytest.mark.parametrize("thomas", ["serial", "partitioned"])
 @pytest.mark.parametrize("resident", [0, 1])
 def test_fused_128_threads_equals_256(thomas, resident):
