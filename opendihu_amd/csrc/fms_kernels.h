@@ -18,7 +18,8 @@
 //                     which follow each other without a solve between them, in
 //                     one pass over the states)
 //   k_reaction_fibre  the same with one workgroup per fibre (large models)
-//   k_thomas_serial   one wave per fibre, the reference's Thomas recurrence (bit-exact)
+//   k_thomas_serial   one wave per fibre, the reference's Thomas recurrence (bit-exact);
+//                     k_thomas_serial_lanes: one lane per fibre, many short fibres
 //   k_thomas_part     one workgroup per fibre, partitioned Thomas + PCR in LDS
 //                     (models of more than 8 states; small models: fms_chunk.h)
 //   k_fused           one workgroup per fibre, many split steps; Vm lives in LDS,
@@ -578,12 +579,23 @@ FMS_HD double div_by(double a, double b, double recip) {
 #endif
 }
 
-// The reference recurrence bit for bit, one wave per fibre: the lanes assemble 64
-// rows at a time, lane 0 runs the recurrence over them (8 rows from LDS to registers
-// at a time, so that only the chain of dependent operations counts: about 12 per row,
-// one division), and the lanes store its results. With one fibre per lane the
-// assembly and its loads stood in the chain, and 1024 fibres filled 16 waves: 315 us
-// per solve of 1024 fibres of 101-301 nodes.
+// The reference recurrence bit for bit, one lane per fibre. A row's assembly, its loads
+// and its division stand in the chain, about 1 us per row, but 64 chains share a wave:
+// for many short fibres (serial_by_lanes).
+static __global__ __launch_bounds__(64) void k_thomas_serial_lanes(DevFibers fb, double *vm, double *cA, double *dA,
+                                                                   StepRef sr, int ie) {
+  const int f = blockIdx.x * blockDim.x + threadIdx.x;
+  if (f >= fb.n_fibers) return;
+  const double dt = sr.row()[3];
+  const int off = fb.fiber_off[f];
+  const int n = fb.fiber_off[f + 1] - off;
+  thomas_serial_fiber(vm + off, n, fb.elem_len + off - f, fb.prefactor[f], dt, ie != 0, cA + off, dA + off);
+}
+
+// The same, one wave per fibre: the lanes assemble 64 rows at a time, lane 0 runs the
+// recurrence over them (8 rows from LDS to registers at a time, so that only the chain
+// of dependent operations counts: about 12 per row, one division), and the lanes store
+// its results. By lanes, 1024 fibres of 101-301 nodes fill 16 waves: 315 us per solve.
 static __global__ __launch_bounds__(64) void k_thomas_serial(DevFibers fb, double *vm, double *cA, double *dA,
                                                              StepRef sr, int ie) {
   __shared__ double ra[64], rb[64], rc[64], rd[64];
@@ -604,9 +616,10 @@ static __global__ __launch_bounds__(64) void k_thomas_serial(DevFibers fb, doubl
     rc[lane] = c;
     rd[lane] = d;
     __syncthreads();
+    const int rows = n - base < 64 ? n - base : 64;
     if (lane == 0) {
-      // rows past the fibre's end are identity rows whose results nobody reads
-      for (int k = 0; k < 64; k += 8) {
+      // the last group's rows past the fibre's end are identity rows whose results nobody reads
+      for (int k = 0; k < rows; k += 8) {
         double va[8], vb[8], vc[8], vd[8];
 #pragma unroll
         for (int q = 0; q < 8; q++) {
@@ -643,8 +656,9 @@ static __global__ __launch_bounds__(64) void k_thomas_serial(DevFibers fb, doubl
     rc[lane] = i < n - 1 ? cA[off + i] : 0.0;   // the last row is its own solution
     rd[lane] = i < n ? dA[off + i] : 0.0;
     __syncthreads();
+    const int rows = n - base < 64 ? n - base : 64;
     if (lane == 0)
-      for (int k = 56; k >= 0; k -= 8) {
+      for (int k = (rows - 1) / 8 * 8; k >= 0; k -= 8) {
         double vc[8], vd[8];
 #pragma unroll
         for (int q = 0; q < 8; q++) {
@@ -663,6 +677,16 @@ static __global__ __launch_bounds__(64) void k_thomas_serial(DevFibers fb, doubl
     if (i < n) u[i] = rd[lane];
     __syncthreads();
   }
+}
+
+// Which of the two: by lanes where there are enough short chains to fill the chip and
+// the lines that neighbouring lanes share stay in the caches until they are read again.
+// us per step of F fibres of n nodes, wave / lanes per fibre: 8192 x 8 21 / 20, 65536 x 10
+// 105 / 60, 262144 x 2 183 / 40, 16384 x 20 49 / 43, 32768 x 24 95 / 91; but
+// 4096 x 10 19 / 21, 8192 x 16 25 / 32, 131072 x 16 216 / 385, 131072 x 24 302 / 574,
+// 32768 x 40 141 / 136 and 16384 x 100 172 / 209.
+inline bool serial_by_lanes(long long n_fibers, int nmax) {
+  return nmax <= 24 && n_fibers >= 8192 && n_fibers >= 800LL * nmax && n_fibers * nmax * nmax <= 25000000LL;
 }
 
 // The same recurrence for many solves with one matrix (fused kernel): what does not

@@ -477,8 +477,12 @@ int launch_thomas(FmsSolver *s, int q) {
     }
   }
   if (s->thomas == FMS_THOMAS_SERIAL) {
-    FMS_LAUNCH(s, fms::k_thomas_serial, dim3(s->F), dim3(64), 0, s->fibers(), s->d_vm, s->d_cA, s->d_dA,
-               step_ref(s, q), ie);
+    if (fms::serial_by_lanes(s->F, s->nmax))
+      FMS_LAUNCH(s, fms::k_thomas_serial_lanes, dim3((s->F + 63) / 64), dim3(64), 0, s->fibers(), s->d_vm, s->d_cA,
+                 s->d_dA, step_ref(s, q), ie);
+    else
+      FMS_LAUNCH(s, fms::k_thomas_serial, dim3(s->F), dim3(64), 0, s->fibers(), s->d_vm, s->d_cA, s->d_dA,
+                 step_ref(s, q), ie);
   } else {
     // rows per chunk: at most ceil(nmax / 256) (>= 3 for fibres under 512 nodes);
     // the smallest register array that holds them

@@ -129,6 +129,20 @@ def test_serial_solve_at_the_edges(kernels):
     np.testing.assert_array_equal(spikes[0], o.spikes()[0])
 
 
+@pytest.mark.parametrize("n_fibers,nmax", [(8191, 8), (8192, 8), (8200, 8), (16384, 16), (25000, 24)])
+def test_serial_solve_of_many_short_fibres(n_fibers, nmax):
+    """one lane or one wave per fibre, whole and partial waves of fibres: the oracle's bits"""
+    n = np.random.default_rng(4).integers(2, nmax + 1, n_fibers)
+    n[0] = nmax
+    mesh = _mesh(n)
+    stim = _pulse(mesh["n_nodes"])
+    rows = _rows(30)
+    o = _oracle(mesh, stim, rows, "CN")
+    states, _ = _run(mesh, stim, rows, scheme="CN", kernels="split", thomas="serial")
+    for k in range(4):
+        np.testing.assert_array_equal(states[k], o.get_state(k), err_msg=f"state {k}")
+
+
 @pytest.mark.parametrize("stim_param,amplitude", [(0, 1200.0), (1, 400.0), (3, 5.0)])
 @pytest.mark.parametrize("n0D", [1, 3])
 def test_pulse_on_any_parameter(stim_param, amplitude, n0D):
