@@ -144,6 +144,16 @@ __device__ __forceinline__ double streamed_half(G *__restrict__ gates, long long
                                        inset, flags, t0, dt, n0D, vstim);
 }
 
+// The serial solve's form (0: the partitioned solve). Small models keep the matrix
+// factored, 5 doubles of LDS per node, unless the flags of a half step's n0D Heun steps
+// leave too little of it: then 2 per node, and thread 0 assembles and factors in each
+// solve. The same bits.
+enum { SERIAL_PLAIN = 1, SERIAL_FACTORED = 2 };
+constexpr size_t FUSED_LDS_BYTES = 160 * 1024;
+inline size_t fused_lds_bytes(int solve_doubles, int nmax, int n0D) {
+  return (size_t)(solve_doubles + 2 * nmax) * sizeof(double) + 2 * (size_t)n0D + 16;
+}
+
 // NPT > 0: gates resident in registers, NPT nodes per thread; NPT == 0: streamed
 template <class M, class G, class E, int T, int MMAX, int NPT>
 __global__ __launch_bounds__(T) void k_fused(DevFibers fb, DevStim st, double *__restrict__ vm,
@@ -159,7 +169,8 @@ __global__ __launch_bounds__(T) void k_fused(DevFibers fb, DevStim st, double *_
   const int n = fb.fiber_off[f + 1] - off;
   const double pf = fb.prefactor[f];
   double *red = sh;   // block interfaces of the partitioned solve, or the serial solve's rows
-  double *lv = sh + (M::NS <= 8 ? serial_lds_doubles(n) : serial ? 16 * T : pcr_lds_doubles<T>());   // n doubles: Vm
+  double *lv = sh + (M::NS <= 8 ? (serial == SERIAL_FACTORED ? serial_lds_doubles(n) : 2 * n)
+                                : serial ? 16 * T : pcr_lds_doubles<T>());   // n doubles: Vm
   double *h = lv + n;   // n - 1 element lengths, staged once for all the launch's solves
   unsigned char *sflags = (unsigned char *)(h + n);   // 2*n0D flags
 
@@ -262,13 +273,13 @@ __global__ __launch_bounds__(T) void k_fused(DevFibers fb, DevStim st, double *_
     const bool more = s + 1 < K;
 
     // diffusion (one solve per split step, as the reference)
-    if constexpr (M::NS <= 8) {   // k_fibre takes these models' partitioned runs
+    if (M::NS <= 8 && serial == SERIAL_FACTORED) {   // k_fibre takes these models' partitioned runs
       if (dt1 != serial_dt) {
         serial_factor(red, n, lv, h, pf, dt1, ie != 0, tid, T);
         serial_dt = dt1;
       }
       serial_solve(red, n, lv, h, pf, dt1, ie != 0, tid, T);
-    } else if (serial) {
+    } else if (M::NS <= 8 || serial) {
       if (tid == 0) thomas_serial_fiber(lv, n, h, pf, dt1, ie != 0, red, red + n);
       __syncthreads();
     } else {

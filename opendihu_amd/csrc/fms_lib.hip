@@ -655,13 +655,20 @@ template <class G, class E, int T, int NPT, int MMAX>
 int launch_fused_npt(FmsSolver *s, const double *d_steps, int K, int n0D, const fms::DevTrace &tr) {
   KernelTimer timer(s, FMS_KERNEL_FUSED);
   const fms::DevSpikes spk = dev_spikes(s);
-  const int red = chunked_model()                   ? fms::serial_lds_doubles(s->nmax)
-                  : s->thomas == FMS_THOMAS_SERIAL ? 16 * T
-                                                   : fms::pcr_lds_doubles<T>();
-  const size_t lds = (size_t)(red + 2 * s->nmax) * sizeof(double) + 2 * (size_t)n0D + 16;
+  int serial = s->thomas == FMS_THOMAS_SERIAL ? fms::SERIAL_PLAIN : 0;
+  int red = serial ? 16 * T : fms::pcr_lds_doubles<T>();
+  if constexpr (chunked_model()) {
+    serial = fms::SERIAL_FACTORED;
+    red = fms::serial_lds_doubles(s->nmax);
+    if (fms::fused_lds_bytes(red, s->nmax, n0D) > fms::FUSED_LDS_BYTES) {
+      serial = fms::SERIAL_PLAIN;
+      red = 2 * s->nmax;
+    }
+  }
+  const size_t lds = fms::fused_lds_bytes(red, s->nmax, n0D);
   FMS_LAUNCH(s, (fms::k_fused<Model, G, E, T, MMAX, NPT>), dim3(s->F), dim3(T), lds, s->fibers(), s->stim(),
              s->d_vm, (G *)s->d_gates, d_steps, K, n0D, s->vstim, s->scheme == FMS_IMPLICIT_EULER ? 1 : 0,
-             s->thomas == FMS_THOMAS_SERIAL ? 1 : 0, s->d_order, spk, tr);
+             serial, s->d_order, spk, tr);
   HIP_TRY(hipGetLastError());
   s->step_counter += K;
   s->n_launch_fused++;

@@ -129,6 +129,21 @@ def test_serial_solve_at_the_edges(kernels):
     np.testing.assert_array_equal(spikes[0], o.spikes()[0])
 
 
+@pytest.mark.parametrize("n,n0D", [(2048, 24350), (2048, 26000), (900, 40000)])
+def test_fused_serial_solve_beside_many_heun_steps(n, n0D):
+    """the flags of a half step's Heun steps share the LDS with the factored matrix (up
+    to 24400 steps at 2048 nodes): past that the solve assembles its rows each time, and
+    the states keep the split kernels' bits"""
+    mesh = _mesh([n, 5])
+    stim = _pulse(mesh["n_nodes"])
+    rows = _rows(1)
+    rows[:, 2] /= n0D
+    fused, _ = _run(mesh, stim, rows, n0D, scheme="CN", kernels="fused", thomas="serial")
+    split, _ = _run(mesh, stim, rows, n0D, scheme="CN", kernels="split", thomas="serial")
+    assert np.isfinite(fused).all() and np.ptp(fused[0]) > 0
+    np.testing.assert_array_equal(fused, split)
+
+
 @pytest.mark.parametrize("n_fibers,nmax", [(8191, 8), (8192, 8), (8200, 8), (16384, 16), (25000, 24)])
 def test_serial_solve_of_many_short_fibres(n_fibers, nmax):
     """one lane or one wave per fibre, whole and partial waves of fibres: the oracle's bits"""
