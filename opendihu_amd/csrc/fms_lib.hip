@@ -680,6 +680,15 @@ size_t fibre_flag_bytes(const FmsSolver *s, int K, int n0D) {
   return (size_t)s->F * fms::flag_groups(K, n0D) * sizeof(fms::FlagGroup);
 }
 
+// Steps of a launch whose flags need not exceed FIBRE_FLAG_BYTES (or one step): with
+// many Heun steps per split step a launch of few steps is long enough, and the flags of
+// 512 would take 256 bytes per fibre and Heun step.
+constexpr size_t FIBRE_FLAG_BYTES = 64 << 20;
+int fibre_launch_steps(const FmsSolver *s, int K, int n0D, size_t bytes) {
+  while (K > 1 && (fibre_flag_bytes(s, K, n0D) > bytes || 2LL * K * n0D > (1 << 30))) K = (K + 1) / 2;
+  return K;
+}
+
 // the flags of K steps, then the steps
 template <class G, class E, bool TAPE>
 int launch_fibre(FmsSolver *s, const double *d_steps, int K, int n0D, const fms::DevTrace &tr) {
@@ -789,12 +798,8 @@ int run(FmsSolver *s, const double *h_steps, int K, int n0D, bool fused_only) {
   int chunk = s->tune_chunk;
   if constexpr (chunked_model() && fms::is_fma<E>::value) {
     // the flags of a launch: allocated, or as many steps as the fixed scratch holds
-    chunk = std::min({chunk, K, std::max(1, (1 << 29) / n0D)});
-    if (!s->noalloc) {
-      if (ensure_flag_bytes(s, fibre_flag_bytes(s, chunk, n0D))) return FMS_ERR_HIP;
-    } else {
-      while (chunk > 1 && fibre_flag_bytes(s, chunk, n0D) > s->flags_cap) chunk = (chunk + 1) / 2;
-    }
+    chunk = fibre_launch_steps(s, std::min(chunk, K), n0D, s->noalloc ? s->flags_cap : FIBRE_FLAG_BYTES);
+    if (!s->noalloc && ensure_flag_bytes(s, fibre_flag_bytes(s, chunk, n0D))) return FMS_ERR_HIP;
   }
   for (int k0 = 0; k0 < K; k0 += chunk) {
     const int kc = std::min(chunk, K - k0);
@@ -1822,7 +1827,7 @@ int adjoint_forward(FmsSolver *s, const double *steps, int n_steps, int n0D, int
   s->adj_interval = Kc;
   // with the whole tape nothing ties a launch to a segment: the solver's
   // steps per fused launch
-  const int len = whole ? s->tune_chunk : Kc;
+  const int len = whole ? fibre_launch_steps(s, std::min(s->tune_chunk, K), n0D, FIBRE_FLAG_BYTES) : Kc;
   if (ensure_flag_bytes(s, fibre_flag_bytes(s, std::min(len, K), n0D))) return FMS_ERR_HIP;
   for (int seg = 0; seg * (long long)len < K; seg++) {
     const int k0 = seg * len, kc = std::min(len, K - k0);

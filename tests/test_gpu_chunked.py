@@ -129,6 +129,25 @@ def test_serial_solve_at_the_edges(kernels):
     np.testing.assert_array_equal(spikes[0], o.spikes()[0])
 
 
+def test_flags_of_many_heun_steps_are_bounded():
+    """a launch covers fewer steps where its flags (16 bytes per fibre and 64 Heun steps)
+    would take more than 64 MiB: 512 steps of 2 x 64 Heun steps are 256 MiB here"""
+    import torch
+    from opendihu_amd.fibers import FiberBatch
+    F, n0D, K = 16384, 64, 512
+    mesh = _mesh(np.full(F, 2))
+    b = FiberBatch(**mesh, scheme="CN", kernels="fused")
+    rows = _rows(K)
+    rows[:, 2] /= n0D
+    b.advance_schedule(rows[:1], n0D)
+    b.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    b.advance_schedule(rows, n0D)
+    b.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= 100 << 20
+    assert b.launch_counts()["fused"] == 1 + 4
+
+
 @pytest.mark.parametrize("n,n0D", [(2048, 24350), (2048, 26000), (900, 40000)])
 def test_fused_serial_solve_beside_many_heun_steps(n, n0D):
     """the flags of a half step's Heun steps share the LDS with the factored matrix (up
