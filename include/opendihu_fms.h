@@ -183,7 +183,8 @@ int fms_last_error(char *buf, int len);
 /* schedule knobs of the fused kernel (the autotuner's search space) */
 #define FMS_TUNE_STEPS_PER_LAUNCH 1   /* split steps per fused launch (default 512) */
 #define FMS_TUNE_RESIDENT_GATES 2     /* -1 auto, 0 stream gates from HBM, 1 keep them in registers;
-                                         small models with the partitioned solve always keep them */
+                                         small models with the partitioned solve always keep them; with
+                                         the serial solve at most 32 per thread are kept, more are streamed */
 /* onlyComputeIfHasBeenStimulated (0/1, default 0): a fibre's reaction runs from
    the Heun step of its first stimulation on; diffusion always runs */
 #define FMS_TUNE_ONLY_IF_STIMULATED 3

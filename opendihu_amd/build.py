@@ -132,6 +132,16 @@ REFERENCE_MODELS = [
 SHORTEN_LIBRARY = "libfms_shorten_ocallaghan_davidson_soboleva_2007.so"
 GEN_HH_LIBRARY = "libfms_gen_hodgkin_huxley_1952.so"
 
+# the generated 8-state model of the tests (tests/eight_state_model.c), the largest that
+# takes the chunked kernels; built wherever the tests are present
+TEST_MODEL = os.path.join(REPO_DIR, "tests", "eight_state_model.c")
+TEST_MODEL_LIBRARY = "libfms_eight_state.so"
+
+
+def build_test_model() -> str:
+    return build_model_library(TEST_MODEL, [], [0, 1, 2, 3], "eight_state", TEST_MODEL_LIBRARY)
+
+
 # Models the reference ships only as hand-written Vc kernels, converted to the
 # OpenCOR form by opendihu_amd.cellml.vc_kernel (no parameters: the kernels
 # take none, stimulation clamps Vm):

@@ -726,6 +726,12 @@ int launch_fibre(FmsSolver *s, const double *d_steps, int K, int n0D, const fms:
   return 0;
 }
 
+// Resident gates: at most 32 doubles (64 registers) of them per thread beside what the
+// reaction and the serial solve need. More, at 8 nodes per thread of an 8-state model,
+// left 256 registers, 230 accumulation registers and 390 spilled scalar ones, and that
+// build lost the eighth node's states (NaN); streamed gates give the split kernels' bits.
+constexpr bool resident_fits(int npt) { return npt * (Model::NS - 1) <= 32; }
+
 // Fused schedules: one workgroup of T threads per fibre; gates resident in
 // registers (NPT nodes per thread, small models) or streamed from HBM. The
 // partitioned solve needs ceil(n / T) <= MMAX rows per thread, the serial
@@ -744,7 +750,8 @@ int launch_fused(FmsSolver *s, const double *d_steps, int K, int n0D, const fms:
       // resident gates for at most 8 nodes per thread: 16 per thread spill to
       // scratch, and that build of the fused kernel computed wrong states
       const int npt = (s->nmax + 127) / 128;
-      if (resident && npt <= 8) return launch_fused_npt<G, E, 128, 8, 8>(s, d_steps, K, n0D, tr);
+      constexpr int NPT = resident_fits(8) ? 8 : 4;
+      if (resident && npt <= NPT) return launch_fused_npt<G, E, 128, NPT, 8>(s, d_steps, K, n0D, tr);
       return launch_fused_npt<G, E, 128, 0, 8>(s, d_steps, K, n0D, tr);
     }
   }
@@ -752,7 +759,8 @@ int launch_fused(FmsSolver *s, const double *d_steps, int K, int n0D, const fms:
   const int npt = (s->nmax + T - 1) / T;
   if constexpr (Model::NS <= 8) {
     if (resident && npt <= 4) return launch_fused_npt<G, E, T, 4, 8>(s, d_steps, K, n0D, tr);
-    if (resident && npt <= 8) return launch_fused_npt<G, E, T, 8, 8>(s, d_steps, K, n0D, tr);
+    if constexpr (resident_fits(8))
+      if (resident && npt <= 8) return launch_fused_npt<G, E, T, 8, 8>(s, d_steps, K, n0D, tr);
   }
   if (npt <= 8) return launch_fused_npt<G, E, T, 0, 8>(s, d_steps, K, n0D, tr);
   return launch_fused_npt<G, E, T, 0, 16>(s, d_steps, K, n0D, tr);

@@ -8,7 +8,8 @@
 * the 57-state TK2014 library (converted from the reference's hand-written Vc
   kernel) must be bit-identical to the oracle's TK2014 model, which takes the
   kernel's lines by another route.
-The generated libraries are built from the reference's CellML inputs where that
+* the kernels of a generated model of 8 states (eight_state_model.c) must agree.
+The other generated libraries are built from the reference's CellML inputs where that
 checkout exists (build()); the tests skip when the library was not built.
 """
 import os
@@ -46,6 +47,45 @@ def test_generated_hh_equals_handwritten():
         b.advance(0.0, 1e-3, 2500)
         runs.append(b.get_states())
     np.testing.assert_array_equal(runs[0], runs[1])
+
+
+# 1 to 8 nodes per thread of 256, 128 and 512 threads; whole and partial last slots
+@pytest.mark.parametrize("lengths,threads", [([2, 5, 200, 257, 700, 1000, 1024], 256), ([300, 1300, 2047, 2048, 65], 256),
+                                             ([2, 100, 129, 513, 900, 1024], 128), ([3000, 4096, 2100], 256)])
+@pytest.mark.parametrize("exp_mode,precision", [("approx", "fp64"), ("libm", "fp64"), ("approx", "mixed")])
+def test_generated_small_model_kernels_agree(lengths, threads, exp_mode, precision):
+    """a generated model of 8 states, the largest on the chunked kernels: with either
+    solve the fused kernels' states have the split kernels' bits, and the partitioned
+    solve's Vm is the serial one's (1e-10; FP32 gates 1e-5)"""
+    from opendihu_amd.build import TEST_MODEL_LIBRARY
+    from opendihu_amd.fibers import FiberBatch
+    lib = _lib_or_skip(TEST_MODEL_LIBRARY)
+    n = np.array(lengths, np.int32)
+    rng = np.random.default_rng(3)
+    mesh = dict(n_nodes=n, element_lengths=0.01 * rng.uniform(0.9, 1.1, int(n.sum()) - n.size),
+                prefactor=rng.uniform(0.006, 0.009, n.size))
+    vm = {}
+
+    def run(kernels, thomas, resident=None):
+        b = FiberBatch(**mesh, scheme="CN", kernels=kernels, thomas=thomas, exp_mode=exp_mode, precision=precision,
+                       library=lib)
+        b.set_tuning(threads=threads)
+        if resident is not None:
+            b.set_tuning(resident_gates=resident)
+        b.set_current_stimulation(np.maximum(n // 2 - 1, 0).astype(np.int32),
+                                  np.minimum(n // 2 + 2, n).astype(np.int32), np.zeros(n.size),
+                                  np.full(n.size, 0.1), np.full(n.size, 3000.0))
+        b.advance(0.0, 2e-3, 60, dt0D=5e-4, n0D=2)
+        return b.get_states()
+
+    for thomas in ("serial", "partitioned"):
+        split = run("split", thomas)
+        vm[thomas] = split[0]
+        assert np.isfinite(split).all() and np.ptp(split[0]) > 50
+        # the fused serial solve takes fibres of up to 2048 nodes
+        for resident in [None] if thomas == "partitioned" else [0, 1] if max(lengths) <= 2048 else []:
+            np.testing.assert_array_equal(run("fused", thomas, resident), split, err_msg=f"{thomas} {resident}")
+    assert _rel(vm["partitioned"], vm["serial"]) <= (1e-10 if precision == "fp64" else 1e-5)
 
 
 def _shorten_pair(kernels, thomas, F=6, n=301, steps=1500, precision="fp64", dt=2e-4, model=SHORTEN):
