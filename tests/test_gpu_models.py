@@ -1,7 +1,9 @@
 """Generated CellML models on the GPU (through the C ABI) against the oracle.
 
 * the Hodgkin-Huxley library generated from the reference's model file must be
-  bit-identical to the hand-written HH library (same expression order);
+  bit-identical to the hand-written HH library (same expression order) with the
+  serial solve, and within 1e-10 (relative L2) of the oracle with the partitioned
+  one, where the hand-written model's reaction takes fused multiply-adds;
 * the 56-state Shorten library must be bit-identical to the oracle's Shorten
   model with the serial Thomas solve, and within 1e-10 (relative L2) with the
   partitioned solve;
@@ -42,11 +44,30 @@ def test_generated_hh_equals_handwritten():
     mesh, stim = uneven(8, lo=300, hi=900, seed=4)
     runs = []
     for name in ("libfms_hodgkin_huxley_1952.so", lib):
-        b = FiberBatch(**mesh, scheme="CN", kernels="fused", library=name)
+        b = FiberBatch(**mesh, scheme="CN", kernels="fused", thomas="serial", library=name)
         b.set_current_stimulation(**stim)
         b.advance(0.0, 1e-3, 2500)
         runs.append(b.get_states())
     np.testing.assert_array_equal(runs[0], runs[1])
+
+
+def test_generated_hh_partitioned():
+    """generated models of at most 8 states on the chunked kernels: the oracle's Vm, and
+    the same bits from the fused and the split kernels"""
+    from opendihu_amd.fibers import FiberBatch
+    lib = _lib_or_skip("libfms_gen_hodgkin_huxley_1952.so")
+    mesh, stim = uneven(8, lo=300, hi=2300, seed=4)
+    o = OracleBatch(**mesh, scheme="CN", threads=8)
+    o.set_current_stimulation(**stim)
+    o.advance(0.0, 1e-3, 1000)
+    runs = []
+    for kernels in ("fused", "split"):
+        b = FiberBatch(**mesh, scheme="CN", kernels=kernels, thomas="partitioned", library=lib)
+        b.set_current_stimulation(**stim)
+        b.advance(0.0, 1e-3, 1000)
+        runs.append(b.get_states())
+    np.testing.assert_array_equal(runs[0], runs[1])
+    assert _rel(runs[0][0], o.vm()) <= 1e-10
 
 
 # 1 to 8 nodes per thread of 256, 128 and 512 threads; whole and partial last slots

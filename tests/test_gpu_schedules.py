@@ -136,12 +136,13 @@ def test_graph_recaptures_when_the_threads_change():
     assert out[1][1]["captures"] == 3
 
 
-@pytest.mark.parametrize("thomas", ["serial", "partitioned"])
-@pytest.mark.parametrize("resident", [0, 1])
+@pytest.mark.parametrize("thomas,resident", [("serial", 0), ("serial", 1), ("partitioned", -1)])
 def test_fused_128_threads_equals_256(thomas, resident):
-    """serial solve: bit-identical; partitioned solve: the partition follows the
-    thread count (another elimination order), so the bar is the partitioned one"""
-    mesh, stim = uneven(10, lo=300, hi=1000 if thomas == "serial" or resident else 2000, seed=8)
+    """serial solve: bit-identical; partitioned solve (its kernel keeps the gates in
+    registers whatever the setting, and takes 128 threads up to 1024 nodes): the
+    partition follows the thread count, so the bar is the partitioned one, and the
+    bits differ"""
+    mesh, stim = uneven(10, lo=300, hi=1000, seed=8)
     runs = []
     for threads in (256, 128):
         g = _batch(mesh, scheme="CN", thomas=thomas, kernels="fused")
@@ -155,7 +156,7 @@ def test_fused_128_threads_equals_256(thomas, resident):
     else:
         err = np.linalg.norm(runs[0][0][0] - runs[1][0][0]) / np.linalg.norm(runs[0][0][0])
         print(f"128 vs 256 threads, partitioned: Vm rel L2 {err:.3e}")
-        assert err <= 1e-10
+        assert 0 < err <= 1e-10
     np.testing.assert_array_equal(runs[0][1][0], runs[1][1][0])
 
 
