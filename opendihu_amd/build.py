@@ -45,7 +45,8 @@ HIP_FLAGS = [
 # scheduler, which is faster for them (occupancy matters there).
 LARGE_MODEL_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 LARGE_MODEL_STATES = 8
-SMALL_MODEL_PARTS = 8   # FMS_PART values of fms_parts.hip
+# FMS_PART values of fms_parts.hip; the last four are the adjoint's (Hodgkin-Huxley only)
+SMALL_MODEL_PARTS, ADJOINT_PARTS = 4, 4
 
 HH_LIBRARY = "libfms_hodgkin_huxley_1952.so"
 
@@ -78,6 +79,8 @@ def compile_library(out_name: str, model_header: str | None = None, model_type: 
     # the host runtime, and the small models' large kernels in objects of their own
     # (fms_parts.h), one compiler process each
     parts = SMALL_MODEL_PARTS if n_states <= LARGE_MODEL_STATES else 0
+    if model_header is None:   # the hand-written model
+        parts += ADJOINT_PARTS
     with tempfile.TemporaryDirectory(dir=LIB_DIR) as tmp:
         jobs = [[os.path.join(CSRC, "fms_lib.hip"), "-o", os.path.join(tmp, "lib.o")]]
         jobs += [[f"-DFMS_PART={k}", os.path.join(CSRC, "fms_parts.hip"), "-o", os.path.join(tmp, f"part{k}.o")]

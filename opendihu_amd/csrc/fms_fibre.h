@@ -1,16 +1,18 @@
 // Resident fused kernel of the small models (at most 8 states, partitioned
-// solve): one workgroup per fibre runs many split steps with the whole state of
-// the fibre in registers.
+// solve): one workgroup per fibre runs many split steps and reads and writes the
+// fibre's state once.
 //
 //  * Thread t owns the c = ceil(n / T) consecutive nodes from t*c on, for the
-//    reaction and for the diffusion (fms_chunk.h) alike: Vm and gates never leave
-//    its registers between two launches, and the diffusion's coefficients stay
-//    beside them as long as dt does not change. One barrier per split step.
+//    reaction and for the diffusion (fms_chunk.h) alike: Vm and gates stay with it
+//    between two launches, and the diffusion's coefficients beside them as long as dt
+//    does not change. One barrier per split step. The kernel is compiled for two waves
+//    per SIMD, 256 registers; with 5 to 8 nodes per thread about 40 values are spilled
+//    to scratch.
 //  * Waves past the fibre's end skip the reaction; threads past it shadow its
 //    last node and store nothing.
-//  * Nodes are advanced two at a time (two independent chains per instruction
-//    stream); the Heun step with a stimulus is a second copy of that code, taken
-//    by the waves that hold stimulated nodes while the stimulus is on.
+//  * Nodes are advanced one after the other (two per basic block gained nothing at two
+//    waves per SIMD); a stimulus's selects stand behind a branch that only the waves
+//    with stimulated nodes take, while the stimulus is on.
 //  * The stimulation state machine does not depend on the states: k_fibre_flags
 //    evaluates it for the whole launch beforehand, one wave per fibre, 64 Heun
 //    steps at a time.
@@ -151,13 +153,13 @@ __device__ __forceinline__ void fibre_heun(double *V, G (*g)[M::NS - 1], const d
     if (!on || st.clamp || st.param == 0) {
       constexpr_for<0, C, 1>([&](auto k_) {
         constexpr int k = decltype(k_)::value;
-        double p0[1] = {p[0]};
-        if (on && !st.clamp) p0[0] = (inset >> k) & 1 ? amplitude : p[0];
-        hh_step_nodes<G, E, false, 1>(V + k, g + k, p, p0, dt,
-                                      [&](double(*ys)[4]) {
-                                        if (on && st.clamp) ys[0][0] = (inset >> k) & 1 ? st.vstim : ys[0][0];
-                                      },
-                                      nullptr);
+        double i_stim = p[0];
+        if (on && !st.clamp) i_stim = (inset >> k) & 1 ? amplitude : p[0];
+        hh_step<G, E, false>(V[k], g[k], p, i_stim, dt,
+                             [&](double &v) {
+                               if (on && st.clamp) v = (inset >> k) & 1 ? st.vstim : v;
+                             },
+                             nullptr);
         if (on && st.clamp) V[k] = (inset >> k) & 1 ? st.vstim : V[k];
       });
       return;
@@ -318,14 +320,9 @@ __device__ __forceinline__ void fibre_steps(const DevFibers &fb, const FibreStim
     }
 }
 
-// waves per SIMD the kernel is compiled for
-template <int T, int CMAX> constexpr int fibre_occupancy() {
-  return T >= 512 && CMAX <= 4 ? 4 : 2;
-}
-
 // one workgroup per fibre; its threads take as many nodes each as the fibre needs
 template <class M, class G, class E, int T, int CMAX, bool TAPE>
-__global__ __launch_bounds__(T, (fibre_occupancy<T, CMAX>())) void k_fibre(
+__global__ __launch_bounds__(T, 2) void k_fibre(
     DevFibers fb, FibreStim st, double *__restrict__ vm, G *__restrict__ gates, const double *__restrict__ steps, int K,
     int n0D, int ie, const int *__restrict__ order, DevSpikes spk, DevTrace tr) {
   extern __shared__ double sh[];

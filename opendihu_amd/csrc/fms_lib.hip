@@ -483,7 +483,7 @@ int launch_thomas(FmsSolver *s, int q) {
     else
       FMS_LAUNCH(s, fms::k_thomas_serial, dim3(s->F), dim3(64), 0, s->fibers(), s->d_vm, s->d_cA, s->d_dA,
                  step_ref(s, q), ie);
-  } else {
+  } else if constexpr (!chunked_model()) {
     // rows per chunk: at most ceil(nmax / 256) (>= 3 for fibres under 512 nodes);
     // the smallest register array that holds them
     const size_t lds = (size_t)(fms::pcr_lds_doubles<PART_T>() + s->nmax) * sizeof(double);
@@ -740,7 +740,7 @@ template <class G, class E>
 int launch_fused(FmsSolver *s, const double *d_steps, int K, int n0D, const fms::DevTrace &tr = fms::DevTrace{}) {
   if constexpr (chunked_model() && fms::is_fma<E>::value) {
     // sensors and the tape are the adjoint's, which runs in FP64
-    if constexpr (std::is_same<G, double>::value)
+    if constexpr (std::is_same<G, double>::value && std::is_same<Model, fms::ModelHH>::value)
       if (tr.sensor_slot || tr.tape) return launch_fibre<G, E, true>(s, d_steps, K, n0D, tr);
     return launch_fibre<G, E, false>(s, d_steps, K, n0D, tr);
   } else {
@@ -762,8 +762,10 @@ int launch_fused(FmsSolver *s, const double *d_steps, int K, int n0D, const fms:
     if constexpr (resident_fits(8))
       if (resident && npt <= 8) return launch_fused_npt<G, E, T, 8, 8>(s, d_steps, K, n0D, tr);
   }
-  if (npt <= 8) return launch_fused_npt<G, E, T, 0, 8>(s, d_steps, K, n0D, tr);
-  return launch_fused_npt<G, E, T, 0, 16>(s, d_steps, K, n0D, tr);
+  // small models come here with the serial solve, of at most 8 rows per thread
+  if constexpr (!chunked_model())
+    if (npt > 8) return launch_fused_npt<G, E, T, 0, 16>(s, d_steps, K, n0D, tr);
+  return launch_fused_npt<G, E, T, 0, 8>(s, d_steps, K, n0D, tr);
   }
 }
 

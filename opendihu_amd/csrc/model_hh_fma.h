@@ -179,48 +179,31 @@ FMS_HD void hh_rates_fused(double V, double m, double h, double n, const double 
   }
 }
 
-// Heun step of Q nodes, as heun_node (fms_kernels.h). STIM: the stimulus may be on:
-// p0[q] holds node q's i_Stim and clamp[q] says whether its Vm is held at vstim;
-// else i_Stim is p[0] on every node. The nodes' chains interleave within each of the
-// three stretches between the stimulus's branches.
-template <class G, class E, bool ALG, int Q, class Clamp>
-FMS_HD void hh_step_nodes(double *V, G (*g)[3], const double *p, const double *p0, double dt, Clamp &&clamp,
-                          double *alg_out) {
-  double r[Q][4], ys[Q][4], rs[Q][4];
+// Heun step of one node, as heun_node (fms_kernels.h), but for the second clamp, which
+// is the caller's. i_stim: the node's i_Stim; clamp(v) holds Vm at the stimulus's value
+// if the step's stimulus does so.
+template <class G, class E, bool ALG, class Clamp>
+FMS_HD void hh_step(double &V, G *g, const double *p, double i_stim, double dt, Clamp &&clamp, double *alg_out) {
+  double r[4], ys[4], rs[4];
+  hh_rates_fused<E, false>(V, (double)g[0], (double)g[1], (double)g[2], p, r, nullptr);
+  r[0] += i_stim;
+  ys[0] = __builtin_fma(dt, r[0], V);
 #pragma unroll
-  for (int q = 0; q < Q; q++) {
-    hh_rates_fused<E, false>(V[q], (double)g[q][0], (double)g[q][1], (double)g[q][2], p, r[q], nullptr);
-    r[q][0] += p0[q];
-    ys[q][0] = __builtin_fma(dt, r[q][0], V[q]);
-#pragma unroll
-    for (int k = 1; k < 4; k++) ys[q][k] = __builtin_fma(dt, r[q][k], (double)g[q][k - 1]);
-  }
-  clamp(ys);
-#pragma unroll
-  for (int q = 0; q < Q; q++) hh_rates_fused<E, ALG>(ys[q][0], ys[q][1], ys[q][2], ys[q][3], p, rs[q], alg_out);
+  for (int k = 1; k < 4; k++) ys[k] = __builtin_fma(dt, r[k], (double)g[k - 1]);
+  clamp(ys[0]);
+  hh_rates_fused<E, ALG>(ys[0], ys[1], ys[2], ys[3], p, rs, alg_out);
   const double hdt = 0.5 * dt;
+  rs[0] += i_stim;
+  V = __builtin_fma(hdt, r[0] + rs[0], V);
 #pragma unroll
-  for (int q = 0; q < Q; q++) {
-    rs[q][0] += p0[q];
-    V[q] = __builtin_fma(hdt, r[q][0] + rs[q][0], V[q]);
-#pragma unroll
-    for (int k = 1; k < 4; k++) g[q][k - 1] = (G)__builtin_fma(hdt, r[q][k] + rs[q][k], (double)g[q][k - 1]);
-  }
+  for (int k = 1; k < 4; k++) g[k - 1] = (G)__builtin_fma(hdt, r[k] + rs[k], (double)g[k - 1]);
 }
 
 // Heun step of one node, as heun_node
 template <class G, class E, bool ALG>
 FMS_HD void hh_step_fused(double &V, G *g, const double *p, double dt, bool clamp, double vstim, double *alg_out) {
-  double v[1] = {V};
-  G gg[1][3] = {{g[0], g[1], g[2]}};
-  hh_step_nodes<G, E, ALG, 1>(v, gg, p, p, dt,
-                              [&](double(*ys)[4]) {
-                                if (clamp) ys[0][0] = vstim;
-                              },
-                              alg_out);
-  V = clamp ? vstim : v[0];
-#pragma unroll
-  for (int k = 0; k < 3; k++) g[k] = gg[0][k];
+  hh_step<G, E, ALG>(V, g, p, p[0], dt, [&](double &v) { if (clamp) v = vstim; }, alg_out);
+  V = clamp ? vstim : V;
 }
 
 }  // namespace fms
