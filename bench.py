@@ -59,8 +59,8 @@ TRAFFIC_FILE = os.path.join(REPO, "profiles", "traffic.json")
 
 def measured_traffic(workload: str, kclass: str, threads: int, nodes: int, node_steps_per_launch: float):
     """(HBM bytes per launch, source) of the dominant kernel from its record
-    (bytes per node and launch, or per node-step for a fused launch of several
-    split steps), or (None, None)"""
+    (bytes per node and launch, or per node-step for a fused launch that streams
+    states in each of its split steps), or (None, None)"""
     try:
         with open(TRAFFIC_FILE) as f:
             for r in json.load(f)["records"]:
@@ -505,7 +505,8 @@ def main(argv=None):
         f_unit = 2 * ops + 5 * g.n_states
         b_unit = bytes_per_node_step(g.n_states, "fp64") / halves
     else:
-        kernel = "k_fused"
+        # the partitioned solve of small models keeps its states in registers
+        kernel = "k_fibre" if g.n_states <= 8 else "k_fused"
         units_per_launch = n_total * prof_steps / max(1, n_launch)
         f_unit = L.flops_per_node_step(g.lib, g.n_states, 1, scheme)
         b_unit = bytes_per_node_step(g.n_states, "fp64")
