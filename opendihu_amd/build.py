@@ -45,8 +45,8 @@ HIP_FLAGS = [
 # scheduler, which is faster for them (occupancy matters there).
 LARGE_MODEL_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]
 LARGE_MODEL_STATES = 8
-# FMS_PART values of fms_parts.hip; the last four are the adjoint's (Hodgkin-Huxley only)
-SMALL_MODEL_PARTS, ADJOINT_PARTS = 4, 4
+# FMS_PART values of fms_parts.hip; the last two are the reverse sweep's (Hodgkin-Huxley only)
+SMALL_MODEL_PARTS, ADJOINT_PARTS = 6, 2
 
 HH_LIBRARY = "libfms_hodgkin_huxley_1952.so"
 

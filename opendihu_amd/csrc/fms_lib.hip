@@ -739,8 +739,8 @@ constexpr bool resident_fits(int npt) { return npt * (Model::NS - 1) <= 32; }
 template <class G, class E>
 int launch_fused(FmsSolver *s, const double *d_steps, int K, int n0D, const fms::DevTrace &tr = fms::DevTrace{}) {
   if constexpr (chunked_model() && fms::is_fma<E>::value) {
-    // sensors and the tape are the adjoint's, which runs in FP64
-    if constexpr (std::is_same<G, double>::value && std::is_same<Model, fms::ModelHH>::value)
+    // sensors and the tape are the adjoint forward's, which runs in FP64 with any model
+    if constexpr (std::is_same<G, double>::value)
       if (tr.sensor_slot || tr.tape) return launch_fibre<G, E, true>(s, d_steps, K, n0D, tr);
     return launch_fibre<G, E, false>(s, d_steps, K, n0D, tr);
   } else {

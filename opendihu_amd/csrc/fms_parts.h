@@ -26,7 +26,7 @@ struct FibreLaunch {
   hipEvent_t start, stop;   // bound to the launch, or null
 };
 
-// T threads per fibre: 128, 256 or 512
+// T threads per fibre: 128, 256 or (without the tape) 512
 template <class G, class E, bool TAPE> void fibre_launch(int T, const FibreLaunch &l);
 
 extern template void fibre_launch<double, ExpApproxFma, false>(int, const FibreLaunch &);

@@ -16,8 +16,10 @@ template <class G, class E, int T, int C, bool TAPE> void fibre_launch_shape(con
 }
 
 template <class G, class E, bool TAPE> void fibre_launch(int T, const FibreLaunch &l) {
+  // 512 threads are for fibres of more than 2048 nodes, which the adjoint does not take
+  if constexpr (!TAPE)
+    if (T == 512) return fibre_launch_shape<G, E, 512, 8, TAPE>(l);
   if (T == 128) fibre_launch_shape<G, E, 128, 8, TAPE>(l);
-  else if (T == 512) fibre_launch_shape<G, E, 512, 8, TAPE>(l);
   else fibre_launch_shape<G, E, 256, 8, TAPE>(l);
 }
 

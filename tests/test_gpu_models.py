@@ -109,6 +109,38 @@ def test_generated_small_model_kernels_agree(lengths, threads, exp_mode, precisi
     assert _rel(vm["partitioned"], vm["serial"]) <= (1e-10 if precision == "fp64" else 1e-5)
 
 
+@pytest.mark.parametrize("thomas", ["serial", "partitioned"])
+@pytest.mark.parametrize("tape", ["whole", "segments"])
+def test_forward_traces_of_a_generated_model(thomas, tape):
+    """sensor traces are recorded with any model (only the reverse sweep is the
+    Hodgkin-Huxley model's): the split kernels' Vm after each step, bit for bit"""
+    from opendihu_amd import _lib as L
+    from opendihu_amd.build import TEST_MODEL_LIBRARY
+    from opendihu_amd.fibers import FiberBatch
+    lib = _lib_or_skip(TEST_MODEL_LIBRARY)
+    n = np.array([5, 300, 1100, 2048], np.int32)
+    mesh = dict(n_nodes=n, element_lengths=np.full(int(n.sum()) - 4, 0.01), prefactor=np.full(4, 0.0077))
+    stim = dict(stim_begin=np.maximum(n // 2 - 1, 0).astype(np.int32), stim_end=(n // 2 + 2).astype(np.int32),
+                onset=np.zeros(4), duration=np.full(4, 0.1), amplitude=np.full(4, 3000.0))
+    sensors = np.ascontiguousarray(np.stack([n // 2 - 2, n // 2, n - 1], 1), np.int32)
+    K = 30
+    rows = np.stack([np.arange(K) * 2e-3, np.full(K, 2e-3), np.full(K, 1e-3), np.full(K, 2e-3)], 1)
+    b = FiberBatch(**mesh, scheme="CN", kernels="fused", thomas=thomas, library=lib)
+    b.set_current_stimulation(**stim)
+    b.set_tuning(adjoint_tape=1 if tape == "whole" else 0)
+    traces = np.full((K, 4, 3), np.nan)
+    L.check(b.lib, b.lib.fms_set_sensors(b.handle, L.as_ptr(sensors, L._ip), 3), "fms_set_sensors")
+    L.check(b.lib, b.lib.fms_adjoint_forward(b.handle, L.as_ptr(rows, L._dp), K, 1, 7, L.as_ptr(traces, L._dp)),
+            "fms_adjoint_forward")
+    s = FiberBatch(**mesh, scheme="CN", kernels="split", thomas=thomas, library=lib)
+    s.set_current_stimulation(**stim)
+    off = np.concatenate([[0], np.cumsum(n)[:-1]])
+    for k in range(K):
+        s.advance_schedule(rows[k:k + 1])
+        np.testing.assert_array_equal(traces[k], s.vm()[off[:, None] + sensors], err_msg=f"step {k}")
+    np.testing.assert_array_equal(b.get_states(), s.get_states())
+
+
 def _shorten_pair(kernels, thomas, F=6, n=301, steps=1500, precision="fp64", dt=2e-4, model=SHORTEN):
     from opendihu_amd.fibers import FiberBatch
     lib = _lib_or_skip(f"libfms_{model}.so")
